@@ -57,7 +57,7 @@ enum { kQKV = 0, kO = 1, kGU = 2, kDN = 3 };
 
 struct PLin {
     const uint8_t *W;        // GPU layout (qlinear.hip), rows padded
-    const float *scales;     // [rows, G]
+    const float *scales;     // [tile][G][16 rows]
     int wld, G, nsteps, rows, tiles, kpad;
 };
 
@@ -121,7 +121,7 @@ EIF_DEV int n_tiles(int tiles) { return tiles > (int)blockIdx.x ? (tiles - 1 - (
 
 // Loader wave: the workgroup's tiles of linear L into its LDS region. Per tile and step one load instruction of SB
 // bytes per lane, laid out as the MFMA lanes read them (lane l: row l & 15, slot l >> 4) at kLdsLane bytes per lane
-// (global_load_lds writes a lane's 12 bytes at a 16-byte lane stride too), then the tile's group scales [16][G] in
+// (global_load_lds writes a lane's 12 bytes at a 16-byte lane stride too), then the tile's group scales [G][16] in
 // 16-byte pieces. Returns the number of load instructions issued.
 template <int SB>
 EIF_DEV int issue_tiles(const PLin L, uint8_t *region, int tile_bytes, int codes_bytes, int tid)
@@ -132,10 +132,10 @@ EIF_DEV int issue_tiles(const PLin L, uint8_t *region, int tile_bytes, int codes
     for (int i = 0; i < nt; ++i) {
         const int tile = (int)blockIdx.x + i * (int)gridDim.x;
         uint8_t *dst = region + i * tile_bytes;
-        const uint8_t *src = L.W + (size_t)(16 * tile + (lane & 15)) * L.wld + (lane >> 4) * SB;
+        const uint8_t *src = L.W + (size_t)tile * (16 * L.wld) + lane * SB;
         for (int st = 0; st < L.nsteps; ++st, ++n) {
-            if constexpr (SB == 16) __builtin_amdgcn_global_load_lds(src + st * 64, dst + st * 64 * kLdsLane, 16, 0, 0);
-            else __builtin_amdgcn_global_load_lds(src + st * 48, dst + st * 64 * kLdsLane, 12, 0, 0);
+            if constexpr (SB == 16) __builtin_amdgcn_global_load_lds(src + st * 64 * SB, dst + st * 64 * kLdsLane, 16, 0, 0);
+            else __builtin_amdgcn_global_load_lds(src + st * 64 * SB, dst + st * 64 * kLdsLane, 12, 0, 0);
         }
         const int pieces = 4 * L.G;   // 16 rows x G floats = 4 G pieces of 16 bytes
         const uint8_t *ssrc = reinterpret_cast<const uint8_t *>(L.scales + (size_t)16 * tile * L.G);
@@ -231,19 +231,20 @@ EIF_DEV void mfma_tiles(const PLin L, int nt, const uint8_t *region, int tile_by
     }
 }
 
-// One row's group combine in group order (qgemv_kernel's step 5): t = fmaf((float)acc_g, s_g, t), y = t * xs.
+// One row's group combine in group order (qgemv_kernel's step 5): t = fmaf((float)acc_g, s_g, t), y = t * xs; the
+// row's scales 16 floats apart.
 EIF_DEV float combine_row(const int32_t *ap, const float *sp, int G, float xs)
 {
     float t = 0.0f;
     int g = 0;
     for (; g + 4 <= G; g += 4) {
         const int4 a4 = *reinterpret_cast<const int4 *>(ap + g);
-        t = fmaf((float)a4.x, sp[g], t);
-        t = fmaf((float)a4.y, sp[g + 1], t);
-        t = fmaf((float)a4.z, sp[g + 2], t);
-        t = fmaf((float)a4.w, sp[g + 3], t);
+        t = fmaf((float)a4.x, sp[16 * g], t);
+        t = fmaf((float)a4.y, sp[16 * (g + 1)], t);
+        t = fmaf((float)a4.z, sp[16 * (g + 2)], t);
+        t = fmaf((float)a4.w, sp[16 * (g + 3)], t);
     }
-    for (; g < G; ++g) t = fmaf((float)ap[g], sp[g], t);
+    for (; g < G; ++g) t = fmaf((float)ap[g], sp[16 * g], t);
     return t * xs;
 }
 
@@ -305,7 +306,7 @@ EIF_DEV void linear_stage(const PArgs &a, int l, uint8_t *smem, PScratch &ps, bo
         const int tt = j >> 4, r = j & 15;
         const int orow = 16 * ((int)blockIdx.x + tt * (int)gridDim.x) + r;
         if (orow < L.rows) {
-            const float *sp = reinterpret_cast<const float *>(region + tt * a.tile_bytes[LI] + a.codes_bytes[LI]) + r * L.G;
+            const float *sp = reinterpret_cast<const float *>(region + tt * a.tile_bytes[LI] + a.codes_bytes[LI]) + r;
             float out = combine_row(acc_l + (tt * 16 + r) * a.gld, sp, L.G, ps.xs_l[0]);
             if constexpr (LI == kO || LI == kDN) out = out + ld_coh(y + orow);
             st_coh(y + orow, out);

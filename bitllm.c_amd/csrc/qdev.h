@@ -36,6 +36,22 @@ struct Geo<kI8, UD> {
     static constexpr int SB = 32, SC = 128, NMF = 4, SHIFT = 0;
 };
 
+// Byte of slot s of `row` at step 0 of a resident weight, and the bytes from one step to the next: ternary rows lie
+// tile-major ([16-row tile][step][slot][row]), INT8 and INT4 row by row.
+template <int FMT, int UD>
+EIF_DEV uint32_t wt_base(int row, int s, int wld)
+{
+    if constexpr (FMT == kTern)
+        return (uint32_t)(row >> 4) * (uint32_t)(16 * wld) + (uint32_t)((16 * s + (row & 15)) * Geo<FMT, UD>::SB);
+    else
+        return (uint32_t)row * (uint32_t)wld + (uint32_t)(s * Geo<FMT, UD>::SB);
+}
+template <int FMT, int UD>
+constexpr int wt_step() { return (FMT == kTern ? 64 : 4) * Geo<FMT, UD>::SB; }
+
+// Group 0's scale of `row` ([16-row tile][group][16 rows]: the next group's is 16 floats on).
+EIF_DEV uint32_t gs_base(int row, int G) { return (uint32_t)(row >> 4) * (uint32_t)(16 * G) + (uint32_t)(row & 15); }
+
 template <int N>
 EIF_DEV void load_words(const uint8_t *p, uint32_t (&w)[N])
 {
