@@ -42,6 +42,7 @@
 
 #include "hip_common.h"
 #include "qdev.h"
+#include "qgemm_tile.h"
 
 namespace {
 
@@ -1516,6 +1517,20 @@ struct FixedWs {
 };
 thread_local FixedWs tl_fixed_ws;
 
+// The stream's split workspace: arrival counters (zeroed when it is allocated), then `bytes` of partial sums. 1 when
+// it cannot be had.
+int split_space(hipStream_t st, size_t bytes, float **part, int **cnt)
+{
+    constexpr size_t cnt_bytes = (size_t)kMaxSplitTiles * sizeof(int);
+    bool fresh = false;
+    float *ws = split_ws(st, cnt_bytes + bytes, 0, &fresh);
+    if (!ws) return 1;
+    *cnt = reinterpret_cast<int *>(ws);
+    *part = ws + kMaxSplitTiles;
+    if (fresh && hipMemsetAsync(*cnt, 0, cnt_bytes, st) != hipSuccess) return EIF_HIP_E_DEVICE;
+    return EIF_HIP_OK;
+}
+
 // Splits along K for `tiles` output tiles of nv values per thread, with the partials' space (ks x tiles x 256
 // threads x nv floats) and the tiles' counters; 1 when the launch is not split.
 template <bool ACC>
@@ -1531,14 +1546,8 @@ int pick_split(QArgs &a, int tiles, int nv, bool grouped, hipStream_t st)
         a.cnt = tl_fixed_ws.cnt;
         return ks;
     }
-    constexpr size_t cnt_bytes = (size_t)kMaxSplitTiles * sizeof(int);
-    bool fresh = false;
-    float *ws = split_ws(st, cnt_bytes + bytes, 0, &fresh);
-    if (!ws) return 1;
-    a.cnt = reinterpret_cast<int *>(ws);
-    a.part = ws + kMaxSplitTiles;
-    if (fresh && hipMemsetAsync(a.cnt, 0, cnt_bytes, st) != hipSuccess) return -2;
-    return ks;
+    const int rc = split_space(st, bytes, &a.part, &a.cnt);
+    return rc == 1 ? 1 : (rc ? -2 : ks);
 }
 
 int g_gemm_pf = 0;   // register buffers of the GEMM's prefetch ring (2, 4, 8), 0 = chosen from the launch
@@ -1630,10 +1639,44 @@ int launch_gemm_t(QArgs a, int rows_pad, hipStream_t st)
     return go(std::integral_constant<int, 2>{});
 }
 
+// The register-tiled form where its rule takes the shape, split along K as the forms below would split it (so that
+// the outputs have the same bits); 1 when it does not, or no workspace for the splits can be had.
+template <int FMT, int UD, bool GROUPED>
+int launch_gemm_large(const QArgs &a, int rows_pad, hipStream_t st)
+{
+    if (FMT != kTern) return 1;
+    eif::TileGemm t{};
+    t.W = a.W, t.scales = a.scales, t.xq = a.xq, t.xs = a.xs, t.bias = a.bias, t.y = a.y;
+    t.fmt = FMT, t.ud = UD, t.grouped = GROUPED, t.wld = a.wld, t.rows_pad = rows_pad, t.G = a.G;
+    t.ldq = a.ldq, t.ldy = a.ldy, t.M = a.M, t.N = a.N, t.nsteps = a.nsteps;
+    const int tt = gemm_tt(a.M, rows_pad / 64, a.nsteps, GROUPED), old_tiles = rows_pad / 64 * eif_ceil_div(a.M, 16 * tt);
+    t.ks = old_tiles > kMaxSplitTiles ? 1 : choose_split(a.nsteps, old_tiles, GROUPED);
+    int tiles = 0;
+    size_t bytes = 0;
+    if (!eif::gemm_tile_takes(t, &tiles, &bytes)) return 1;
+    if (t.ks > 1) {
+        if (tiles > kMaxSplitTiles) return 1;
+        if (tl_fixed_ws.ptr) {   // what the forms below refuse for its splits is left to them to refuse
+            const size_t old_bytes = (size_t)t.ks * old_tiles * kGemmThreads * 4 * tt * sizeof(float);
+            if (std::max(bytes, old_bytes) > tl_fixed_ws.bytes) return 1;
+            t.part = tl_fixed_ws.ptr, t.cnt = tl_fixed_ws.cnt;
+        } else {
+            const int rc = split_space(st, bytes, &t.part, &t.cnt);
+            if (rc) return rc;
+        }
+    }
+    return eif::launch_gemm_tile(t, st);
+}
+
 // Token tile of the GEMM: 16, 32 or 64 tokens (gemm_tt).
 template <int FMT, int UD, bool GROUPED, bool ACC>
 int launch_gemm(const QArgs &a, int rows_pad, hipStream_t st)
 {
+    // large batches: the register-tiled form (qgemm_tile.hip), unless a knob asks for one of the forms here
+    if (!ACC && g_gemm_tt == 0 && g_gemm_split == 0 && g_gemm_pf == 0 && g_gemm_panel == 0) {
+        const int rc = launch_gemm_large<FMT, UD, GROUPED>(a, rows_pad, st);
+        if (rc != 1) return rc;
+    }
     switch (gemm_tt(a.M, rows_pad / 64, a.nsteps, GROUPED)) {
     case 1: return launch_gemm_t<FMT, UD, GROUPED, ACC, 1>(a, rows_pad, st);
     case 2: return launch_gemm_t<FMT, UD, GROUPED, ACC, 2>(a, rows_pad, st);

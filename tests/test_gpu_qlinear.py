@@ -682,3 +682,45 @@ def test_rowpair_gemv(gpu, oracle, fmt, N, K, mode):
     finally:
         lib.eif_hip_set_gemv_rowpair(old)
     qw.close()
+
+
+@pytest.mark.parametrize("N,K,g,M", [
+    # the register-tiled form from one 32-token x 128-row workgroup per CU on: 256 or more here, so its small shape
+    (130, 200, 32, 4100),      # rows past 128 and short of 192, a ragged last step
+    (128, 96, 96, 8161),       # one step; one token past whole blocks
+    (1000, 500, 64, 1025),     # ragged rows and columns
+    (1100, 2560, 128, 1000),
+    (700, 600, 256, 1376),     # an odd count of groups
+    (960, 864, 96, 1100),      # whole groups, an odd count
+    # its large shape (64 tokens x 256 rows), from 384 such workgroups on
+    (300, 160, 32, 12300),
+    (6912, 300, 128, 899),
+    (2560, 672, 96, 2449),     # rows of whole blocks; g96, a step and a half
+    (3000, 320, 64, 2050),
+    (520, 1100, 256, 8200),
+    # one scale per row: small from 160 workgroups on, then large
+    (1300, 700, 0, 500),
+    (129, 256, 0, 5121),
+    (520, 260, 0, 8200),
+])
+def test_gemm_tile(gpu, oracle, N, K, g, M):
+    """The register-tiled GEMM: outputs bit for bit those of the oracle (group sums combined in group order, exact
+    int32 sums over K with row scales), with a bias or none, in rows of a wider y whose other columns stay as they are."""
+    import torch
+    w, s = synth.ternary_weight((80, N, K, g), N, K, g)
+    x = synth.activations((81, M, K), M, K, outliers=False)
+    qw = gpu.QWeight(gpu.W_TERNARY, N, K, g, w, s)
+    xq, xs, xq_d, xs_d = dev_inputs(gpu, oracle, x, qw.kpad)
+    for bias in (None, synth.rng(82, N).standard_normal(N).astype(np.float32)):
+        oy = np.zeros((M, N), np.float32)
+        if g:
+            oracle.orc_ternary_gemv_grouped(P(w), P(s), g, P(xq), qw.kpad, P(xs), P(bias), P(oy), N, M, N, K)
+        else:
+            oracle.orc_ternary_gemv_rowscale(P(w), P(s), P(xq), qw.kpad, P(xs), P(bias), P(oy), N, M, N, K)
+        yd = torch.full((M, N + 3), 7.0, dtype=torch.float32, device="cuda:0")
+        b = torch.from_numpy(bias).to("cuda:0") if bias is not None else None
+        qw.linear(xq_d, xs_d, yd, bias=b, path=GEMM)
+        y = yd.cpu().numpy()
+        assert np.array_equal(y[:, :N].view(np.uint32), oy.view(np.uint32)), bias is None
+        assert np.all(y[:, N:] == 7.0)
+    qw.close()
