@@ -483,6 +483,21 @@ def test_prefill_long_split(gpu, oracle):
     check_prefill(gpu, oracle, cfg, w, prompt, [100, 100])
 
 
+@pytest.mark.parametrize("heads,kv,hd,chunks", [
+    (4, 4, 32, [17]),          # one query head a kv head: four 32-query blocks a workgroup; just past the 16-token form
+    (4, 2, 64, [33, 31]),      # two heads, two blocks; a second batch at a position inside a tile
+    (6, 2, 64, [40]),          # three heads, a spare wave
+    (5, 1, 32, [65]),          # five heads: a second workgroup of one head
+    (8, 1, 128, [32, 16, 64]), # eight heads; whole tiles; the 16-token form between
+    (4, 1, 128, [160, 33]),    # ranges of more than one share
+])
+def test_prefill_attention_shapes(gpu, oracle, heads, kv, hd, chunks):
+    cfg = synth.bitnet_config(min(256, heads * hd), 384, 2, heads, kv, hd, 500, 200, 32, 32, 32, 32, 128)
+    w = synth.bitnet_model((28, heads, kv, hd), cfg)
+    prompt = list(np.random.default_rng(29).integers(0, cfg["vocab"], sum(chunks) + 1))
+    check_prefill(gpu, oracle, cfg, w, prompt, chunks)
+
+
 def test_prefill_then_greedy(gpu, oracle):
     cfg, w = tiny()
     prompt = list(np.random.default_rng(7).integers(0, cfg["vocab"], 12))
