@@ -41,6 +41,7 @@
 #include <unordered_map>
 
 #include "hip_common.h"
+#include "prep_batch.h"
 #include "qdev.h"
 #include "qgemm_tile.h"
 
@@ -2210,6 +2211,8 @@ int launch_prep_spec(PrepArgs p, int8_t *xq, int ldq, float *xs, int M, hipStrea
 {
     if (!xq || !xs || ldq < p.K || ldq % 16 != 0 || ((uintptr_t)xq & 15) || M < 1) return EIF_HIP_E_ARG;
     p.ldl = ldq;
+    const int rc = eif::launch_prep_batch({p.x, p.ldx, p.signs, p.nw, p.K, p.block, p.norm, p.eps, p.pre, xq, ldq, xs, M}, st);
+    if (rc != 1) return rc;
     for (int e = 4; e <= 16; e *= 2) {
         if (64 * e < p.block || eif_ceil_div(ldq, e) > 1024) continue;
         if (e == 4) return launch_prep_spec_e<4>(p, xq, xs, M, st);

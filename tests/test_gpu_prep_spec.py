@@ -202,3 +202,39 @@ def test_glu_form(gpu, oracle, N, K, M):
     assert lib.eif_hip_qlinear_prep_glu(q3.h, C.byref(sp), gpu.ptr(yg), h, M, gpu.stream_ptr()) == -4   # LIMIT
     for q in (qw, qd, q3):
         q.close()
+
+
+@pytest.mark.parametrize("K,ldq,block,pre,signs", [
+    (32, 32, 32, 1, True),        # one chunk of columns, mostly empty
+    (512, 528, 64, 0, False),     # a whole chunk, padding in the next one
+    (544, 768, 0, 1, False),
+    (2080, 2304, 32, 1, True),
+    (2560, 2560, 128, 1, True),   # the BitNet layer inputs
+    (2560, 2560, 128, 0, True),
+    (3072, 3072, 256, 1, False),
+    (4096, 4096, 128, 1, True),   # the longest row it takes
+])
+def test_prep_batch_rows(gpu, K, ldq, block, pre, signs):
+    """Batches of 768 rows and more (one wave a row): codes and scales bit for bit those of smaller batches (one
+    workgroup a row), zeros past K, a row of zeros among them."""
+    import torch
+    dev = torch.device("cuda:0")
+    M = 771
+    x = torch.from_numpy(synth.activations((90, K), M, K)).to(dev)
+    x[5] = 0.0
+    nw = torch.from_numpy((1.0 + 0.1 * synth.rng(91, K).standard_normal(K)).astype(np.float32)).to(dev)
+    sg = torch.from_numpy(np.where(synth.rng(92, K).random(K) < 0.5, -1.0, 1.0).astype(np.float32)).to(dev) if signs else None
+
+    def prep(lo, hi):
+        xq = torch.full((hi - lo, ldq), 99, dtype=torch.int8, device=dev)
+        xs = torch.full((hi - lo,), -1.0, dtype=torch.float32, device=dev)
+        sp = gpu.prep_spec(x[lo:hi], pre, None, nw, 1e-5, sg, block, gpu.wht_norm(block) if block else 1.0)
+        gpu.prep_spec_rows(sp, K, xq, xs, hi - lo)
+        torch.cuda.synchronize()
+        return xq.cpu().numpy(), xs.cpu().numpy()
+
+    q, s = prep(0, M)
+    parts = [prep(0, 400), prep(400, M)]
+    assert np.array_equal(q, np.concatenate([p[0] for p in parts]))
+    assert np.array_equal(s.view(np.uint32), np.concatenate([p[1] for p in parts]).view(np.uint32))
+    assert not q[:, K:].any() and not q[5].any() and s[5] == 1.0
