@@ -700,6 +700,17 @@ int enqueue_prefill(eif_hip_bitnet *m, int pos0, int n, hipStream_t st)
         if (rc) return rc;
         return eif_hip_qlinear_ex(w, m->p_xq, kp, m->p_xs, nullptr, y, ldy, n, EIF_HIP_PATH_AUTO, st);
     };
+    // x += linear(prep(sp)): in the GEMM's epilogue where its form allows, else through p_y
+    auto prep_linear_add = [&](const eif_hip_qweight *w, const eif_hip_prep_spec &sp, int K) -> int {
+        const int kp = kpad_of(w);
+        int rc = eif_hip_prep_spec_rows(&sp, K, m->p_xq, kp, m->p_xs, n, st);
+        if (rc) return rc;
+        if ((rc = eif::qlinear_add(w, m->p_xq, kp, m->p_xs, m->p_x, c.dim, n, st)) != 1) return rc;
+        if ((rc = eif_hip_qlinear_ex(w, m->p_xq, kp, m->p_xs, nullptr, m->p_y, c.dim, n, EIF_HIP_PATH_AUTO, st))) return rc;
+        add_rows_kernel<<<add_blocks, 256, 0, st>>>(m->p_x, m->p_y, (size_t)n * c.dim);
+        EIF_HIP_LAUNCHED();
+        return EIF_HIP_OK;
+    };
     embed_rows_kernel<<<n, 256, 0, st>>>(m->emb, m->emb_scale, m->prompt, pos0, m->p_x, c.dim);
     EIF_HIP_LAUNCHED();
     for (int l = 0; l < c.n_layers; ++l) {
@@ -738,9 +749,7 @@ int enqueue_prefill(eif_hip_bitnet *m, int pos0, int n, hipStream_t st)
         sp = eif_hip_prep_spec{};
         sp.x = m->p_xb, sp.ldx = m->q_dim, sp.pre = EIF_HIP_PRE_RMS, sp.norm_w = m->rms_sub_att[l];
         sp.eps = c.sub_eps, sp.signs = m->signs_q, sp.wht_block = c.wht_q, sp.wht_norm = c.wht_norm_q;
-        if ((rc = prep_linear(m->wo[l], sp, m->q_dim, m->p_y, c.dim))) return rc;
-        add_rows_kernel<<<add_blocks, 256, 0, st>>>(m->p_x, m->p_y, (size_t)n * c.dim);   // x += O xb
-        EIF_HIP_LAUNCHED();
+        if ((rc = prep_linear_add(m->wo[l], sp, m->q_dim))) return rc;   // x += O xb
         sp = eif_hip_prep_spec{};
         sp.x = m->p_x, sp.ldx = c.dim, sp.pre = EIF_HIP_PRE_RMS, sp.norm_w = m->rms_ffn[l], sp.eps = c.rms_eps;
         sp.signs = m->signs_dim, sp.wht_block = c.wht_dim, sp.wht_norm = c.wht_norm_dim;
@@ -749,9 +758,7 @@ int enqueue_prefill(eif_hip_bitnet *m, int pos0, int n, hipStream_t st)
         sp.x = m->p_h, sp.x2 = m->p_h + c.hidden, sp.ldx = 2 * c.hidden, sp.pre = EIF_HIP_PRE_SWIGLU_RMS;
         sp.norm_w = m->rms_sub_ffn[l], sp.eps = c.sub_eps;
         sp.signs = m->signs_hidden, sp.wht_block = c.wht_hidden, sp.wht_norm = c.wht_norm_hidden;
-        if ((rc = prep_linear(m->w2[l], sp, c.hidden, m->p_y, c.dim))) return rc;
-        add_rows_kernel<<<add_blocks, 256, 0, st>>>(m->p_x, m->p_y, (size_t)n * c.dim);   // x += W2 h
-        EIF_HIP_LAUNCHED();
+        if ((rc = prep_linear_add(m->w2[l], sp, c.hidden))) return rc;   // x += W2 h
     }
     EIF_HIP_TRY(hipMemcpyAsync(m->x, m->p_x + (size_t)(n - 1) * c.dim, sizeof(float) * c.dim,
                                hipMemcpyDeviceToDevice, st));

@@ -99,6 +99,8 @@ int launch_quant_rows(const float *x, int ldx, int M, int K, int8_t *xq, int ldq
 
 int qlinear_scaled(const eif_hip_qweight *w, const float *scales, const int8_t *xq, int ldq, const float *xs,
                    const float *bias, float *y, int ldy, int M, int path, hipStream_t st);
+int qlinear_add(const eif_hip_qweight *w, const int8_t *xq, int ldq, const float *xs, float *x, int ldx, int M,
+                hipStream_t st);
 int qweight_row_tiles(const eif_hip_qweight *w);
 // The GPU layout of a resident weight (qlinear.hip): codes W (rows padded to 64, wld bytes per row; ternary rows in
 // 16-row tiles), scales ([rows / 16][G][16] grouped, [rows] row-scaled or NULL), format, group (0: row-scaled), steps of the layout along K.

@@ -1643,13 +1643,13 @@ int launch_gemm_t(QArgs a, int rows_pad, hipStream_t st)
 // The register-tiled form where its rule takes the shape, split along K as the forms below would split it (so that
 // the outputs have the same bits); 1 when it does not, or no workspace for the splits can be had.
 template <int FMT, int UD, bool GROUPED>
-int launch_gemm_large(const QArgs &a, int rows_pad, hipStream_t st)
+int launch_gemm_large(const QArgs &a, int rows_pad, hipStream_t st, const float *res = nullptr, int ldr = 0)
 {
     if (FMT != kTern) return 1;
     eif::TileGemm t{};
     t.W = a.W, t.scales = a.scales, t.xq = a.xq, t.xs = a.xs, t.bias = a.bias, t.y = a.y;
     t.fmt = FMT, t.ud = UD, t.grouped = GROUPED, t.wld = a.wld, t.rows_pad = rows_pad, t.G = a.G;
-    t.ldq = a.ldq, t.ldy = a.ldy, t.M = a.M, t.N = a.N, t.nsteps = a.nsteps;
+    t.ldq = a.ldq, t.ldy = a.ldy, t.M = a.M, t.N = a.N, t.nsteps = a.nsteps, t.res = res, t.ldr = ldr;
     const int tt = gemm_tt(a.M, rows_pad / 64, a.nsteps, GROUPED), old_tiles = rows_pad / 64 * eif_ceil_div(a.M, 16 * tt);
     t.ks = old_tiles > kMaxSplitTiles ? 1 : choose_split(a.nsteps, old_tiles, GROUPED);
     int tiles = 0;
@@ -2384,6 +2384,29 @@ int qlinear_prep_shares(const eif_hip_qweight *w, const eif_hip_prep_spec *spec,
     a.ldy = ldy;
     rc = dispatch<false>(w, a, p, EIF_HIP_PATH_GEMV, st);
     return rc == 1 ? EIF_HIP_E_LIMIT : rc;
+}
+
+// x += linear of a prepped batch, the sum in the GEMM's epilogue; 1 (nothing launched) where the batch does not take
+// the register-tiled form.
+int qlinear_add(const eif_hip_qweight *w, const int8_t *xq, int ldq, const float *xs, float *x, int ldx, int M, hipStream_t st)
+{
+    int rc = check_linear_args(w, xq, ldq, M);
+    if (rc) return rc;
+    if (!xs || !x || ldx < w->rows) return EIF_HIP_E_ARG;
+    if (w->fmt != kTern || M <= 2 * kGemvTileM || resolve_path(w, EIF_HIP_PATH_AUTO, M) != EIF_HIP_PATH_GEMM ||
+        g_gemm_tt || g_gemm_split || g_gemm_pf || g_gemm_panel)
+        return 1;
+    QArgs a = make_args(w, xq, ldq, M);
+    a.xs = xs, a.y = x, a.ldy = ldx;
+    if (w->group == 0) return launch_gemm_large<kTern, 4, false>(a, w->rows_pad, st, x, ldx);
+    switch (w->ud) {
+    case 1: return launch_gemm_large<kTern, 1, true>(a, w->rows_pad, st, x, ldx);
+    case 2: return launch_gemm_large<kTern, 2, true>(a, w->rows_pad, st, x, ldx);
+    case 3: return launch_gemm_large<kTern, 3, true>(a, w->rows_pad, st, x, ldx);
+    case 4: return launch_gemm_large<kTern, 4, true>(a, w->rows_pad, st, x, ldx);
+    case 8: return launch_gemm_large<kTern, 8, true>(a, w->rows_pad, st, x, ldx);
+    default: return 1;
+    }
 }
 
 // The linear with an explicit scale array (the host drop-in passes per-call row scales for resident codes).
