@@ -673,7 +673,7 @@ __global__ __launch_bounds__(1024) void qgemv_kernel(const void *__restrict__ r0
     const int r16 = lane & 15, s = lane >> 4;
     const int row0 = rb * TR;
     constexpr int RH = RT / 2;   // GLU: gate tiles per workgroup
-    const int glu_t = GLU ? (i1 & 0x7FFFFFF) : 0;   // GLU: tiles of one half
+    const int glu_t = GLU ? (E == 0 ? a.nrb : i1 & 0x7FFFFFF) : 0;   // GLU: tiles of one half
     const int row = GLU ? (rt < RH ? rb * RH + rt : glu_t + rb * RH + rt - RH) * 16 + r16 : row0 + 16 * rt + r16;
     const int kpad = nsteps * GE::SC;
     const int nj = (nsteps - kw + ks - 1) / ks;
@@ -1816,11 +1816,13 @@ int launch_glu_s(const QArgs &a, const PrepArgs &p, int half, int ks, hipStream_
 {
     const size_t lds = gemv_lds_bytes(true, true, a, p.ldl, kGluRT, ks);
     GemvHot h;
-    if (!gemv_hot(a, p, true, false, ks, &h, OPS)) return EIF_HIP_E_LIMIT;
-    h.i1 |= half / 16;   // bits 0..26: the tiles of one half
+    if (!gemv_hot(a, p, E > 0, false, ks, &h, OPS)) return EIF_HIP_E_LIMIT;
+    QArgs ag = a;
+    if constexpr (E > 0) h.i1 |= half / 16;   // bits 0..26: the tiles of one half
+    else ag.nrb = half / 16;
     qgemv_kernel<kTern, 4, true, false, E, SPW, LB, kGluRT, 1, false, true, OPS>
         <<<half / (16 * kGluRT / 2), 64 * kGluRT * ks, lds, st>>>(
-        h.r0, h.r1, h.r2, h.r3, a.W, a.wld, a.nsteps, h.i0, h.i1, a, p);
+        h.r0, h.r1, h.r2, h.r3, a.W, a.wld, a.nsteps, h.i0, h.i1, ag, p);
     EIF_HIP_LAUNCHED();
     return EIF_HIP_OK;
 }
@@ -1828,7 +1830,7 @@ int launch_glu_s(const QArgs &a, const PrepArgs &p, int half, int ks, hipStream_
 template <int E, int LB, int OPS = kOpsAny>
 int launch_glu_e(const QArgs &a, const PrepArgs &p, int half, int ks, hipStream_t st)
 {
-    if constexpr (LB == 7 && OPS == kOpsAny) {   // the BitNet rotation: the operand set compiled in
+    if constexpr (E > 0 && LB == 7 && OPS == kOpsAny) {   // the BitNet rotation: the operand set compiled in
         const float *mul = nullptr;
         const int ops = gemv_ops(p, &mul);
         if (ops == kOpsX) return launch_glu_e<E, LB, kOpsX>(a, p, half, ks, st);
@@ -2126,12 +2128,14 @@ int launch_gemv(const QArgs &a, const PrepArgs &p, int rows_pad, const uint8_t *
     return 1;
 }
 
+constexpr int kPathGemvOnly = 100;   // the GEMV, or 1 where it does not stage the shape
+
 template <int FMT, int UD, bool GROUPED, bool ACC>
 int launch_shape(const QArgs &a, const PrepArgs &p, int rows_pad, int path, hipStream_t st, const uint8_t *wt = nullptr)
 {
-    if (p.x || (path == EIF_HIP_PATH_GEMV && a.M <= kGemvMaxM)) {
+    if (p.x || ((path == EIF_HIP_PATH_GEMV || path == kPathGemvOnly) && a.M <= kGemvMaxM)) {
         const int rc = launch_gemv<FMT, UD, GROUPED, ACC>(a, p, rows_pad, wt, st);
-        if (rc != 1) return rc;
+        if (rc != 1 || path == kPathGemvOnly) return rc;
     }
     return launch_gemm<FMT, UD, GROUPED, ACC>(a, rows_pad, st);
 }
@@ -2429,6 +2433,40 @@ int qlinear_scaled(const eif_hip_qweight *w, const float *scales, const int8_t *
 
 }  // namespace eif
 
+// From kPrepOnceRows token rows on, a linear of FP32 rows preps them in a launch of their own, into the stream's prep
+// workspace, and the GEMV stages the int8 rows: fused, every workgroup preps the rows one after the other (the linears of a
+// BitNet-2B layer, us, fused / prepped: 2 rows 32.3 / 33, 3 rows 41.8 / 33.7, 4 rows 50.9 / 34.0, 8 rows 86.9 / 35.6; the
+// INT4 feed-forward and 151936x1024 head at 3 rows 41.2 / 28.4, at 8 rows 82.1 / 31.8). A short row's prep is a shorter
+// chain, so matrices of up to 1024 columns below the vocabulary sizes go over from kPrepOnceShort rows on (the linears of
+// an INT8 Qwen2.5-0.5B-shaped layer at 3 rows 24.4 / 32.7, at 6 rows 37.5 / 32.5). Codes, scales and sums are the
+// same. 1 (and the fused form is taken) when there is no workspace (a stream's first use inside a capture) or the GEMV
+// does not stage the shape.
+constexpr int kPrepOnceRows = 3, kPrepOnceShort = 5;
+
+static int prep_once(const eif_hip_qweight *w, const PrepArgs &p, QArgs *a, hipStream_t st)
+{
+    const bool brief = w->kpad <= 1024 && w->rows_pad / 16 < kBigTiles;
+    if (a->M < (brief ? kPrepOnceShort : kPrepOnceRows) || !gemv_fits_tile(w)) return 1;
+    const size_t qb = (size_t)a->M * w->kpad;   // a multiple of 16
+    int8_t *xq = reinterpret_cast<int8_t *>(split_ws(st, qb + 4 * (size_t)a->M, 1));
+    if (!xq) return 1;
+    float *xs = reinterpret_cast<float *>(xq + qb);
+    const int rc = launch_prep_spec(p, xq, w->kpad, xs, a->M, st);
+    if (rc) return rc == EIF_HIP_E_LIMIT ? 1 : rc;
+    a->xq = xq, a->ldq = w->kpad, a->xs = xs;
+    return EIF_HIP_OK;
+}
+
+// A linear of at most kFusedMaxM FP32 rows.
+static int linear_rows(const eif_hip_qweight *w, const PrepArgs &p, const QArgs &a, hipStream_t st)
+{
+    QArgs b = a;
+    int rc = prep_once(w, p, &b, st);
+    if (rc == EIF_HIP_OK) rc = dispatch<false>(w, b, PrepArgs{}, kPathGemvOnly, st);
+    if (rc != 1) return rc;
+    return dispatch<false>(w, a, p, EIF_HIP_PATH_GEMV, st);
+}
+
 extern "C" int eif_hip_qlinear_f32(const eif_hip_qweight *w, const float *x, int ldx, const float *signs,
                                    int wht_block, float norm, const float *bias, float *y, int ldy, int M,
                                    void *stream)
@@ -2441,7 +2479,7 @@ extern "C" int eif_hip_qlinear_f32(const eif_hip_qweight *w, const float *x, int
     a.bias = bias;
     a.y = y;
     a.ldy = ldy;
-    return dispatch<false>(w, a, p, EIF_HIP_PATH_GEMV, (hipStream_t)stream);
+    return linear_rows(w, p, a, (hipStream_t)stream);
 }
 
 // More than kFusedMaxM rows of a spec: the prep on its own into the stream's prep workspace (xq [M, kpad], then xs
@@ -2491,7 +2529,7 @@ extern "C" int eif_hip_qlinear_prep(const eif_hip_qweight *w, const eif_hip_prep
             if (rc != 1) return rc;
         }
     }
-    return dispatch<false>(w, a, p, EIF_HIP_PATH_GEMV, st);
+    return linear_rows(w, p, a, st);
 }
 
 // y[m, r] = SiLU(gate_r) * up_r for r < rows / 2 (gate = rows 0 .. rows/2 - 1 of w, up = the rest), one GEMV launch
@@ -2514,6 +2552,17 @@ extern "C" int eif_hip_qlinear_prep_glu(const eif_hip_qweight *w, const eif_hip_
     const int kpad = a.nsteps * Geo<kTern, 4>::SC, maxks = 16 / kGluRT;
     int ks = std::min(g_gemv_ksplit > 0 ? g_gemv_ksplit : eif_ceil_div(a.nsteps, 4), maxks);   // as launch_gemv_tiles
     const hipStream_t st = (hipStream_t)stream;
+    if (M >= kPrepOnceRows && kpad <= 8192) {   // what the fused form takes: up to 8 columns on 1024 threads
+        QArgs b = a;
+        int k = ks;
+        while (k < maxks && (M * (kpad / 16) > kMaxPieces * 64 * kGluRT * k || a.G > gemv_scl<kTern, 4, true>() * 4 * k)) ++k;
+        if (M * (kpad / 16) <= kMaxPieces * 64 * kGluRT * k && a.G <= gemv_scl<kTern, 4, true>() * 4 * k &&
+            gemv_lds_bytes(true, true, a, p.ldl, kGluRT, k) <= gemv_max_lds() && prep_once(w, p, &b, st) == EIF_HIP_OK) {
+            PrepArgs pb{};
+            pb.ldl = p.ldl;
+            return launch_glu_e<0, 0>(b, pb, half, k, st);
+        }
+    }
     for (int e = 4; e <= 8; e *= 2) {
         if (64 * e < p.block || e < g_gemv_prep_cols) continue;
         int k = ks;

@@ -106,8 +106,9 @@ int eif_hip_qlinear_acc(const eif_hip_qweight *w, const int8_t *xq, int ldq, int
 
 /* Prep fused into the GEMV: y = linear(prep(x)) for M <= 8 FP32 rows x [M, ldx] of K = cols (K % 32 == 0,
  * rows and signs 16-byte aligned, ldx % 4 == 0, K <= 16384), with the prep contract above (signs, wht_block <= 1024,
- * norm). One launch; the result equals eif_hip_prep_rows followed by eif_hip_qlinear bit for bit. M > 8
- * returns EIF_HIP_E_LIMIT (use the two calls).                                                         */
+ * norm). One launch (from 3 or 5 rows on, by shape, a prep launch into a per-stream workspace and the GEMV, which is
+ * faster; one launch there too on a stream whose first such call is inside a graph capture); the result equals
+ * eif_hip_prep_rows followed by eif_hip_qlinear bit for bit. M > 8 returns EIF_HIP_E_LIMIT (use the two calls). */
 int eif_hip_qlinear_f32(const eif_hip_qweight *w, const float *x, int ldx, const float *signs, int wht_block,
                         float norm, const float *bias, float *y, int ldy, int M, void *stream);
 int eif_hip_qlinear_f32_acc(const eif_hip_qweight *w, const float *x, int ldx, const float *signs, int wht_block,
@@ -136,8 +137,8 @@ typedef struct eif_hip_prep_spec {
 } eif_hip_prep_spec;
 
 /* eif_hip_qlinear_f32 with a pre-op: y = linear(prep(pre(x))) (+ bias). M <= 8 rows: one launch (a row-scaled
- * matrix of 65536 rows or more at M = 1, e.g. a vocabulary head: a prep launch, then the GEMV of the prepped row,
- * with the same output bits); the bias may then be the residual stream itself (y == bias: each output reads its
+ * matrix of 65536 rows or more at M = 1, e.g. a vocabulary head, and from 3 or 5 rows on as eif_hip_qlinear_f32: a
+ * prep launch, then the GEMV of the prepped rows, with the same output bits); the bias may then be the residual stream itself (y == bias: each output reads its
  * own bias element first). More rows (a prompt batch): the prep of eif_hip_prep_spec_rows into a per-stream
  * workspace, then eif_hip_qlinear on the auto path (the GEMV or the int8-MFMA GEMM by token count and shape),
  * the same bits as those two calls; the bias must not overlap y, and a stream's first such call must be made
