@@ -17,7 +17,7 @@
 // 0 .. 3, i = 0 .. 3), and the staged values are laid out in that order of keys. The four waves of a workgroup are the
 // query heads of a kv head (or more queries of it) on the same staged keys and values.
 //
-// Measured (us a layer, 20 query and 5 kv heads of 128, both kernels of it): 1900 tokens 389 on FP32 MFMAs, 101 here;
+// Measured (us a layer, 20 query and 5 kv heads of 128, both kernels of it): 1900 tokens 389 on FP32 MFMAs, 111 here;
 // 1024 142, 52; 511 50, 31; 256 29, 20; 64 14.4, 10.6; 900 at position 1100 314, 84. Up to 16 tokens, one block of the FP32
 // kernel, that one is ahead (16 tokens 6.9 against 7.8) and stays (decode.hip).
 #include <algorithm>
@@ -234,18 +234,11 @@ void attn_prefill_kernel(eif::PrefillAttn a, int heads_wg, int qb, int ct, int s
 }
 
 // Blocks whose causal range was split: out = sum_s e^(m_s - M) O_s / sum_s e^(m_s - M) l_s over the block's shares,
-// M = max_s m_s (a share with m_s = -inf weighs 0). HD / 4 threads a row (token, head), four dims each, so that a wave
-// reads whole rows of the shares. (One workgroup of HD threads a row, a
-// float each, at 1900 tokens and 20 heads of 128: 22.4 us, 12.3 so.)
-constexpr int kCombineThreads = 256;
-
+// M = max_s m_s (a share with m_s = -inf weighs 0). Workgroup (token i, head), HD threads.
 template <int HD>
-__global__ __launch_bounds__(kCombineThreads) void attn_prefill_combine_kernel(eif::PrefillAttn a, int qb, int ct, int s_call)
+__global__ __launch_bounds__(128) void attn_prefill_combine_kernel(eif::PrefillAttn a, int qb, int ct, int s_call)
 {
-    constexpr int TPR = HD / 4;
-    const int idx = blockIdx.x * (kCombineThreads / TPR) + (int)threadIdx.x / TPR, d = 4 * ((int)threadIdx.x % TPR);
-    if (idx >= a.n * a.n_heads) return;
-    const int i = idx / a.n_heads, h = idx - i * a.n_heads, rows = 32 * qb;
+    const int i = blockIdx.x, h = blockIdx.y, d = threadIdx.x, rows = 32 * qb;
     const int b = i / rows, row = i - rows * b;
     const int all_tiles = (a.pos0 + min(rows * (b + 1), a.n) + kKeys - 1) / kKeys;
     if (all_tiles <= ct) return;   // written by the attention kernel
@@ -253,17 +246,15 @@ __global__ __launch_bounds__(kCombineThreads) void attn_prefill_combine_kernel(e
     const size_t e0 = ((size_t)b * s_call * a.n_heads + h) * rows + row, es = (size_t)a.n_heads * rows;
     float mx = -INFINITY;
     for (int s = 0; s < ns; ++s) mx = fmaxf(mx, a.pml[2 * (e0 + s * es)]);
-    float os[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ls = 0.0f;
+    float os = 0.0f, ls = 0.0f;
     for (int s = 0; s < ns; ++s) {
         const size_t e = e0 + s * es;
-        const float2 ml = *reinterpret_cast<const float2 *>(a.pml + 2 * e);
-        const float4 o = *reinterpret_cast<const float4 *>(a.po + e * HD + d);
-        const float wgt = ml.x == -INFINITY ? 0.0f : expf(ml.x - mx);
-        os[0] = fmaf(wgt, o.x, os[0]), os[1] = fmaf(wgt, o.y, os[1]);
-        os[2] = fmaf(wgt, o.z, os[2]), os[3] = fmaf(wgt, o.w, os[3]);
-        ls = fmaf(wgt, ml.y, ls);
+        const float ms = a.pml[2 * e];
+        const float wgt = ms == -INFINITY ? 0.0f : expf(ms - mx);
+        os = fmaf(wgt, a.po[e * HD + d], os);
+        ls = fmaf(wgt, a.pml[2 * e + 1], ls);
     }
-    *reinterpret_cast<float4 *>(a.out + (size_t)i * a.ldo + h * HD + d) = make_float4(os[0] / ls, os[1] / ls, os[2] / ls, os[3] / ls);
+    a.out[(size_t)i * a.ldo + h * HD + d] = os / ls;
 }
 
 // Query heads and 32-query sub-blocks of a workgroup's four waves: heads of one kv head share its staged keys and
@@ -308,8 +299,7 @@ int launch(const eif::PrefillAttn &a, hipStream_t st)
     attn_prefill_kernel<HD><<<dim3(cols, nblk * s_call), 256, 0, st>>>(a, hw, qb, ct, s_call, 1.0f / sqrtf((float)HD));
     EIF_HIP_LAUNCHED();
     if (s_call > 1) {
-        const int rows_wg = kCombineThreads / (HD / 4);
-        attn_prefill_combine_kernel<HD><<<eif_ceil_div(a.n * a.n_heads, rows_wg), kCombineThreads, 0, st>>>(a, qb, ct, s_call);
+        attn_prefill_combine_kernel<HD><<<dim3(a.n, a.n_heads), HD, 0, st>>>(a, qb, ct, s_call);
         EIF_HIP_LAUNCHED();
     }
     return EIF_HIP_OK;
