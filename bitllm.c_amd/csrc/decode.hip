@@ -21,7 +21,6 @@
 
 #include "hip_common.h"
 #include "attn_dev.h"
-#include "attn_prefill.h"
 #include "persist.h"
 #include "../../include/eif_hip_decode.h"
 
@@ -155,7 +154,7 @@ __global__ __launch_bounds__(256) void rope_append_kernel(float *qkv, int ldqkv,
     }
 }
 
-// Prefill, step 2, batches of up to kPrefillSmall tokens (more: attn_prefill.hip): causal attention of the batch on fp32 MFMAs (v_mfma_f32_16x16x4f32: lane l supplies A[l % 16][l / 16]
+// Prefill, step 2: causal attention of the batch on fp32 MFMAs (v_mfma_f32_16x16x4f32: lane l supplies A[l % 16][l / 16]
 // and B[l / 16][l % 16], and holds D[4 (l / 16) + i][l % 16] in register i). Workgroup (x, y) takes batch tokens
 // [16 b, 16 b + 16) (b = y / s_call) and up to four query heads of kv head g = x / P (P = ceil(kv_mul / 4)), one
 // wave per head, over key tiles [kPrefillTiles s, kPrefillTiles (s + 1)) (s = y % s_call) of the block's causal
@@ -166,7 +165,6 @@ __global__ __launch_bounds__(256) void rope_append_kernel(float *qkv, int ldqkv,
 // whose range is one workgroup's writes out = O / l; a longer one writes each workgroup's share (O, m, l) to
 // po / pml for attn_prefill_combine_kernel.
 constexpr int kPrefillTiles = 8;
-constexpr int kPrefillSmall = 16;
 
 template <int HD>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *qkv, int ldqkv, const __half *kc,
@@ -468,8 +466,7 @@ struct eif_hip_bitnet {
     int pf_cap = 0;
     float *p_x = nullptr, *p_xb = nullptr, *p_qkv = nullptr, *p_h = nullptr, *p_y = nullptr, *p_xs = nullptr;
     float *p_po = nullptr, *p_pml = nullptr;   // attention shares of split blocks [block][share][head][16][HD | 2]
-    int pf_scap = 0;                           // shares per block of a batch of up to kPrefillSmall tokens
-    size_t pf_shares = 0;                      // rows of shares the buffers hold
+    int pf_scap = 0;                           // shares per block the buffers hold
     int8_t *p_xq = nullptr;
     size_t weight_bytes = 0;
     hipGraph_t graph = nullptr;
@@ -647,7 +644,7 @@ void free_prefill(eif_hip_bitnet *m)
                     (void *)m->p_xs, (void *)m->p_xq})
         if (p) (void)hipFree(p);
     m->p_x = m->p_xb = m->p_qkv = m->p_h = m->p_y = m->p_xs = m->p_po = m->p_pml = nullptr;
-    m->pf_scap = 0, m->pf_shares = 0;
+    m->pf_scap = 0;
     m->p_xq = nullptr;
     m->pf_cap = 0;
 }
@@ -670,16 +667,14 @@ int ensure_prefill(eif_hip_bitnet *m, int n)
         free_prefill(m);
         return EIF_HIP_E_NOMEM;
     }
-    // attention shares: up to ceil(ceil(seq_len / 16) / kPrefillTiles) of one 16-token block, and what attn_prefill.hip
-    // asks for (at least as many: its blocks are of 32 tokens or more)
+    // attention shares: up to ceil(ceil(seq_len / 16) / kPrefillTiles) per 16-token block
     const int scap = ((c.seq_len + 15) / 16 + kPrefillTiles - 1) / kPrefillTiles;
-    const size_t ne = std::max((size_t)scap * c.n_heads * 16, eif::prefill_attn_shares(n, c.n_heads, c.n_kv_heads, c.seq_len));
+    const size_t ne = (size_t)((n + 15) / 16) * scap * c.n_heads * 16;
     if (scap > 1 && (hipMalloc(&m->p_po, sizeof(float) * ne * c.head_dim) != hipSuccess ||
                      hipMalloc(&m->p_pml, sizeof(float) * ne * 2) != hipSuccess)) {
         free_prefill(m);
         return EIF_HIP_E_NOMEM;
     }
-    m->pf_shares = scap > 1 ? ne : 0;
     m->pf_scap = scap;
     m->pf_cap = n;
     return EIF_HIP_OK;
@@ -725,25 +720,19 @@ int enqueue_prefill(eif_hip_bitnet *m, int pos0, int n, hipStream_t st)
         rope<<<n, 256, 0, st>>>(m->p_qkv, ldqkv, m->kc + cache_l, m->vc + cache_l, pos0, c.n_heads, c.n_kv_heads,
                                 c.seq_len, m->rope);
         EIF_HIP_LAUNCHED();
-        if (n > kPrefillSmall) {
-            const eif::PrefillAttn pa{m->p_qkv, ldqkv, m->kc + cache_l, m->vc + cache_l, m->p_xb, m->q_dim, m->p_po, m->p_pml,
-                                      m->pf_shares, pos0, n, c.n_heads, c.n_kv_heads, c.seq_len, c.head_dim};
-            if ((rc = eif::launch_attn_prefill(pa, st))) return rc;
-        } else {
-            auto attn = c.head_dim == 128 ? attn_prefill_kernel<128>
-                        : (c.head_dim == 64 ? attn_prefill_kernel<64> : attn_prefill_kernel<32>);
-            const int kv_mul = c.n_heads / c.n_kv_heads, parts = (kv_mul + 3) / 4;
-            const int s_call = ((pos0 + n + 15) / 16 + kPrefillTiles - 1) / kPrefillTiles;   // shares of the longest block
-            attn<<<dim3(c.n_kv_heads * parts, (n + 15) / 16 * s_call), 64 * std::min(kv_mul, 4), 0, st>>>(
-                m->p_qkv, ldqkv, m->kc + cache_l, m->vc + cache_l, m->p_xb, m->q_dim, m->p_po, m->p_pml, s_call,
-                m->pf_scap, pos0, n, c.n_heads, c.n_kv_heads, c.seq_len, inv_sqrt_hd);
-            EIF_HIP_LAUNCHED();
-            if (s_call > 1) {
-                auto comb = c.head_dim == 128 ? attn_prefill_combine_kernel<128>
-                            : (c.head_dim == 64 ? attn_prefill_combine_kernel<64> : attn_prefill_combine_kernel<32>);
-                comb<<<dim3(n, c.n_heads), c.head_dim, 0, st>>>(m->p_po, m->p_pml, m->p_xb, m->q_dim, m->pf_scap, pos0, n,
-                                                                c.n_heads);
-            }
+        auto attn = c.head_dim == 128 ? attn_prefill_kernel<128>
+                    : (c.head_dim == 64 ? attn_prefill_kernel<64> : attn_prefill_kernel<32>);
+        const int kv_mul = c.n_heads / c.n_kv_heads, parts = (kv_mul + 3) / 4;
+        const int s_call = ((pos0 + n + 15) / 16 + kPrefillTiles - 1) / kPrefillTiles;   // shares of the longest block
+        attn<<<dim3(c.n_kv_heads * parts, (n + 15) / 16 * s_call), 64 * std::min(kv_mul, 4), 0, st>>>(
+            m->p_qkv, ldqkv, m->kc + cache_l, m->vc + cache_l, m->p_xb, m->q_dim, m->p_po, m->p_pml, s_call,
+            m->pf_scap, pos0, n, c.n_heads, c.n_kv_heads, c.seq_len, inv_sqrt_hd);
+        EIF_HIP_LAUNCHED();
+        if (s_call > 1) {
+            auto comb = c.head_dim == 128 ? attn_prefill_combine_kernel<128>
+                        : (c.head_dim == 64 ? attn_prefill_combine_kernel<64> : attn_prefill_combine_kernel<32>);
+            comb<<<dim3(n, c.n_heads), c.head_dim, 0, st>>>(m->p_po, m->p_pml, m->p_xb, m->q_dim, m->pf_scap, pos0, n,
+                                                            c.n_heads);
         }
         EIF_HIP_LAUNCHED();
         sp = eif_hip_prep_spec{};

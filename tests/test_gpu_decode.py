@@ -484,11 +484,11 @@ def test_prefill_long_split(gpu, oracle):
 
 
 @pytest.mark.parametrize("heads,kv,hd,chunks", [
-    (4, 4, 32, [17]),          # one query head a kv head: four 32-query blocks a workgroup; just past the 16-token form
-    (4, 2, 64, [33, 31]),      # two heads, two blocks; a second batch at a position inside a tile
-    (6, 2, 64, [40]),          # three heads, a spare wave
+    (4, 4, 32, [17]),          # one query head a kv head; one token past a block
+    (4, 2, 64, [33, 31]),      # two heads; a second batch at a position inside a tile
+    (6, 2, 64, [40]),          # three heads
     (5, 1, 32, [65]),          # five heads: a second workgroup of one head
-    (8, 1, 128, [32, 16, 64]), # eight heads; whole tiles; the 16-token form between
+    (8, 1, 128, [32, 16, 64]), # eight heads; whole tiles
     (4, 1, 128, [160, 33]),    # ranges of more than one share
 ])
 def test_prefill_attention_shapes(gpu, oracle, heads, kv, hd, chunks):
@@ -496,6 +496,43 @@ def test_prefill_attention_shapes(gpu, oracle, heads, kv, hd, chunks):
     w = synth.bitnet_model((28, heads, kv, hd), cfg)
     prompt = list(np.random.default_rng(29).integers(0, cfg["vocab"], sum(chunks) + 1))
     check_prefill(gpu, oracle, cfg, w, prompt, chunks)
+
+
+def test_prefill_infinite_key(gpu, oracle):
+    """Keys that overflow the fp16 cache: one dimension of three layer-0 keys is infinite, so a query's score with such
+    a key is an infinity of the sign of the product. Where it is -inf the key weighs 0 and the row stays that of the
+    other keys: layer 1's keys and values, formed from it, agree with the oracle's. (Those positions: where the
+    oracle's step is the same bits with 1e30 in place of the infinity.)"""
+    cfg = synth.bitnet_config(256, 384, 2, 2, 1, 128, 500, 64, 32, 32, 32, 32, 128)
+    w = synth.bitnet_model((31, 3), cfg)
+    w["gk"][3] *= 74193.89   # row 3 of layer 0's key matrix
+    n = 40
+    prompt = list(np.random.default_rng(35).integers(0, cfg["vocab"], n + 1))
+    m = gpu.BitnetModel(cfg, w)
+    orc = OracleRun(oracle, cfg, w)
+    try:
+        m.reset(prompt)
+        m.prefill(n)
+        kv = [m.kv_cache(layer, 0, n) for layer in range(2)]
+    finally:
+        m.close()
+    first = int(np.argmax(np.isinf(kv[0][0]).any(1)))
+    assert np.isinf(kv[0][0][first, 3]) and np.isinf(kv[0][0]).sum() == 3
+    checked = 0
+    for p in range(n):
+        steps = []
+        for big in (1e30, np.inf):
+            k0 = kv[0][0][:p]
+            orc.kc[0, :p], orc.vc[0, :p] = np.where(np.isinf(k0), np.copysign(np.float32(big), k0), k0), kv[0][1][:p]
+            orc.step(prompt[p], p)
+            steps.append(np.concatenate([orc.kc[1, p], orc.vc[1, p]]))
+        if p <= first or np.isinf(kv[0][0][p]).any() or not np.array_equal(steps[0], steps[1]):
+            continue
+        checked += 1
+        got = np.concatenate([kv[1][0][p], kv[1][1][p]])
+        err = np.abs(got - steps[1]).max() / np.abs(steps[1]).max()
+        assert err <= REL, (p, err)
+    assert checked >= 3, checked
 
 
 def test_prefill_then_greedy(gpu, oracle):
