@@ -2557,10 +2557,13 @@ extern "C" int eif_hip_qlinear_prep_glu(const eif_hip_qweight *w, const eif_hip_
         int k = ks;
         while (k < maxks && (M * (kpad / 16) > kMaxPieces * 64 * kGluRT * k || a.G > gemv_scl<kTern, 4, true>() * 4 * k)) ++k;
         if (M * (kpad / 16) <= kMaxPieces * 64 * kGluRT * k && a.G <= gemv_scl<kTern, 4, true>() * 4 * k &&
-            gemv_lds_bytes(true, true, a, p.ldl, kGluRT, k) <= gemv_max_lds() && prep_once(w, p, &b, st) == EIF_HIP_OK) {
-            PrepArgs pb{};
-            pb.ldl = p.ldl;
-            return launch_glu_e<0, 0>(b, pb, half, k, st);
+            gemv_lds_bytes(true, true, a, p.ldl, kGluRT, k) <= gemv_max_lds()) {
+            if ((rc = prep_once(w, p, &b, st)) == EIF_HIP_OK) {
+                PrepArgs pb{};
+                pb.ldl = p.ldl;
+                return launch_glu_e<0, 0>(b, pb, half, k, st);
+            }
+            if (rc != 1) return rc;
         }
     }
     for (int e = 4; e <= 8; e *= 2) {
