@@ -1433,6 +1433,61 @@ float *split_ws(hipStream_t st, size_t bytes, int slot = 0, bool *fresh = nullpt
     return w.first;
 }
 
+// The int8 rows and scales of a call of up to kFusedMaxM rows that preps them in a launch of its own (prep_once): one
+// buffer per (device, stream), large enough for every such call, so that it never moves. A call holds `mu` while it issues
+// its two launches: calls of several threads on one stream then follow each other in the stream's order. No buffer inside a
+// capture (replays of a graph run beside other work of its stream and would share it), on hipStreamPerThread (one handle, a
+// stream per thread), once kRowsWsMax streams have one, or where it cannot be allocated: the caller takes its single
+// launch there. The buffers (8.4 MB at most) are freed with the last resident weight.
+constexpr size_t kRowsWsBytes = kFusedMaxM * (16384 + sizeof(float));
+constexpr int kRowsWsMax = 64;
+struct RowsWs {
+    int dev;
+    hipStream_t st;
+    int8_t *p;
+    std::mutex mu;
+};
+std::mutex g_rows_mu;   // of what follows
+RowsWs g_rows[kRowsWsMax];
+int g_nrows, g_nweights;
+
+RowsWs *rows_ws(hipStream_t st)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    int dev = 0;
+    if (st == hipStreamPerThread) return nullptr;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
+        (void)hipGetLastError();   // the single launch meets and reports what is wrong with the stream
+        return nullptr;
+    }
+    if (cs != hipStreamCaptureStatusNone) return nullptr;
+    std::lock_guard<std::mutex> lk(g_rows_mu);
+    for (int i = 0; i < g_nrows; ++i)
+        if (g_rows[i].dev == dev && g_rows[i].st == st) return &g_rows[i];
+    if (g_nrows == kRowsWsMax) return nullptr;
+    void *p = nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // an allocation must not end another stream's capture
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const bool ok = hipMalloc(&p, kRowsWsBytes) == hipSuccess;
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ok) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    RowsWs &w = g_rows[g_nrows++];
+    w.dev = dev, w.st = st, w.p = static_cast<int8_t *>(p);
+    return &w;
+}
+
+void count_weight(int d)
+{
+    std::lock_guard<std::mutex> lk(g_rows_mu);
+    g_nweights += d;
+    if (g_nweights > 0) return;
+    for (int i = 0; i < g_nrows; ++i) (void)hipFree(g_rows[i].p);   // waits for launches that still use it
+    g_nrows = 0;
+}
+
 int device_cus()
 {
     static const int n = [] {
@@ -2433,36 +2488,37 @@ int qlinear_scaled(const eif_hip_qweight *w, const float *scales, const int8_t *
 
 }  // namespace eif
 
-// From kPrepOnceRows token rows on, a linear of FP32 rows preps them in a launch of their own, into the stream's prep
-// workspace, and the GEMV stages the int8 rows: fused, every workgroup preps the rows one after the other (the linears of a
+// From kPrepOnceRows token rows on, a linear of FP32 rows preps them in a launch of their own, into the stream's rows
+// buffer, and the GEMV stages the int8 rows: fused, every workgroup preps the rows one after the other (the linears of a
 // BitNet-2B layer, us, fused / prepped: 2 rows 32.3 / 33, 3 rows 41.8 / 33.7, 4 rows 50.9 / 34.0, 8 rows 86.9 / 35.6; the
 // INT4 feed-forward and 151936x1024 head at 3 rows 41.2 / 28.4, at 8 rows 82.1 / 31.8). A short row's prep is a shorter
 // chain, so matrices of up to 1024 columns below the vocabulary sizes go over from kPrepOnceShort rows on (the linears of
 // an INT8 Qwen2.5-0.5B-shaped layer at 3 rows 24.4 / 32.7, at 6 rows 37.5 / 32.5). Codes, scales and sums are the
-// same. 1 (and the fused form is taken) when there is no workspace (a stream's first use inside a capture) or the GEMV
-// does not stage the shape.
+// same. gemv(a) launches the GEMV of the prepped rows, or returns 1 where it does not stage the shape; 1 (and the caller
+// takes the fused form) for that, for fewer rows, and where rows_ws() has no buffer.
 constexpr int kPrepOnceRows = 3, kPrepOnceShort = 5;
 
-static int prep_once(const eif_hip_qweight *w, const PrepArgs &p, QArgs *a, hipStream_t st)
+template <class F>
+static int prep_once(const eif_hip_qweight *w, const PrepArgs &p, QArgs a, hipStream_t st, F gemv)
 {
     const bool brief = w->kpad <= 1024 && w->rows_pad / 16 < kBigTiles;
-    if (a->M < (brief ? kPrepOnceShort : kPrepOnceRows) || !gemv_fits_tile(w)) return 1;
-    const size_t qb = (size_t)a->M * w->kpad;   // a multiple of 16
-    int8_t *xq = reinterpret_cast<int8_t *>(split_ws(st, qb + 4 * (size_t)a->M, 1));
-    if (!xq) return 1;
-    float *xs = reinterpret_cast<float *>(xq + qb);
-    const int rc = launch_prep_spec(p, xq, w->kpad, xs, a->M, st);
+    if (a.M < (brief ? kPrepOnceShort : kPrepOnceRows) || !gemv_fits_tile(w)) return 1;
+    const size_t qb = (size_t)a.M * w->kpad;   // a multiple of 16
+    if (qb + 4 * (size_t)a.M > kRowsWsBytes) return 1;
+    RowsWs *ws = rows_ws(st);
+    if (!ws) return 1;
+    std::lock_guard<std::mutex> lk(ws->mu);
+    float *xs = reinterpret_cast<float *>(ws->p + qb);
+    const int rc = launch_prep_spec(p, ws->p, w->kpad, xs, a.M, st);
     if (rc) return rc == EIF_HIP_E_LIMIT ? 1 : rc;
-    a->xq = xq, a->ldq = w->kpad, a->xs = xs;
-    return EIF_HIP_OK;
+    a.xq = ws->p, a.ldq = w->kpad, a.xs = xs;
+    return gemv(a);
 }
 
 // A linear of at most kFusedMaxM FP32 rows.
 static int linear_rows(const eif_hip_qweight *w, const PrepArgs &p, const QArgs &a, hipStream_t st)
 {
-    QArgs b = a;
-    int rc = prep_once(w, p, &b, st);
-    if (rc == EIF_HIP_OK) rc = dispatch<false>(w, b, PrepArgs{}, kPathGemvOnly, st);
+    const int rc = prep_once(w, p, a, st, [&](const QArgs &b) { return dispatch<false>(w, b, PrepArgs{}, kPathGemvOnly, st); });
     if (rc != 1) return rc;
     return dispatch<false>(w, a, p, EIF_HIP_PATH_GEMV, st);
 }
@@ -2553,16 +2609,15 @@ extern "C" int eif_hip_qlinear_prep_glu(const eif_hip_qweight *w, const eif_hip_
     int ks = std::min(g_gemv_ksplit > 0 ? g_gemv_ksplit : eif_ceil_div(a.nsteps, 4), maxks);   // as launch_gemv_tiles
     const hipStream_t st = (hipStream_t)stream;
     if (M >= kPrepOnceRows && kpad <= 8192) {   // what the fused form takes: up to 8 columns on 1024 threads
-        QArgs b = a;
         int k = ks;
         while (k < maxks && (M * (kpad / 16) > kMaxPieces * 64 * kGluRT * k || a.G > gemv_scl<kTern, 4, true>() * 4 * k)) ++k;
         if (M * (kpad / 16) <= kMaxPieces * 64 * kGluRT * k && a.G <= gemv_scl<kTern, 4, true>() * 4 * k &&
             gemv_lds_bytes(true, true, a, p.ldl, kGluRT, k) <= gemv_max_lds()) {
-            if ((rc = prep_once(w, p, &b, st)) == EIF_HIP_OK) {
+            rc = prep_once(w, p, a, st, [&](const QArgs &b) {
                 PrepArgs pb{};
                 pb.ldl = p.ldl;
                 return launch_glu_e<0, 0>(b, pb, half, k, st);
-            }
+            });
             if (rc != 1) return rc;
         }
     }
@@ -2816,6 +2871,7 @@ int eif_hip_qweight_create(eif_hip_qweight **out, int fmt, int rows, int cols, i
         if (q.tm) (void)hipFree(q.tm);
         return EIF_HIP_E_NOMEM;
     }
+    count_weight(1);
     *out = h;
     return EIF_HIP_OK;
 }
@@ -2827,6 +2883,7 @@ void eif_hip_qweight_destroy(eif_hip_qweight *w)
     if (w->scales) (void)hipFree(w->scales);
     if (w->tm) (void)hipFree(w->tm);
     delete w;
+    count_weight(-1);
 }
 
 int eif_hip_qweight_info(const eif_hip_qweight *w, int *rows, int *cols, int *kpad, int *group, size_t *bytes)

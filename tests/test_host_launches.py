@@ -72,3 +72,67 @@ def test_gated_call_reports_a_failed_prep_launch(fake):
         assert lib.eif_hip_qlinear_prep_glu(w.h, C.byref(spec(K)), X, N // 2, 4, None) == DEVICE
         assert fake.fake_launches() == 1
     """)
+
+
+ROWS_CALLS = """
+    N, K = 512, 2560
+    w = weight(N, K)
+
+    def rows(call, M, st=None):
+        assert call(w, N, K, M, st) == 0
+        return fake.fake_launches(), fake.fake_launch_arg1(0)
+"""
+
+
+def test_rows_calls_in_a_capture_are_one_launch(fake):
+    """3 to 8 rows: a prep launch and the GEMV outside a capture; inside one the single launch, also on a stream that
+    has a rows buffer, and nothing is allocated."""
+    run(fake, ROWS_CALLS + """
+    for call in (linear, glu):
+        for M in (3, 8):
+            for st in (None, 0x100):
+                assert rows(call, M, st)[0] == 2
+                n = fake.fake_mallocs()
+                fake.fake_capturing(1)
+                assert rows(call, M, st)[0] == 1 and rows(call, M, 0x200)[0] == 1 and fake.fake_mallocs() == n
+                fake.fake_capturing(0)
+    """)
+
+
+def test_rows_buffers(fake):
+    """One rows buffer a device and stream, which stays where it is; none for the handle that means a stream per thread;
+    64 at most; all given back with the last resident weight."""
+    run(fake, ROWS_CALLS + """
+    w2 = weight(256, 4096)
+    live = fake.fake_live()
+    _, p = rows(linear, 3)
+    assert fake.fake_live() == live + 1
+    assert linear(w2, 256, 4096, 8) == 0 and fake.fake_launches() == 2 and fake.fake_launch_arg1(0) == p
+    assert rows(glu, 5)[1] == p and rows(linear, 8, 0x100)[1] != p and fake.fake_live() == live + 2
+    fake.fake_device(1)
+    assert rows(linear, 4)[1] not in (p, None) and fake.fake_live() == live + 3
+    fake.fake_device(0)
+    assert rows(linear, 4) == (2, p)
+    assert rows(linear, 4, 2)[0] == 1   # hipStreamPerThread
+    for st in range(0x200, 0x200 + 100):
+        assert rows(linear, 4, st)[0] in (1, 2)
+    assert fake.fake_live() == live + 64 and rows(linear, 4)[0] == 2 and rows(linear, 4, 0x300)[0] == 1
+    w2.close()
+    assert rows(linear, 4) == (2, p)
+    w.close()
+    assert fake.fake_live() == 0
+    w = weight(N, K)
+    assert rows(linear, 4, 0x300)[0] == 2
+    """)
+
+
+def test_rows_call_without_memory(fake):
+    """Where the rows buffer cannot be allocated the call is the single launch, as for one row, and reports no error."""
+    run(fake, ROWS_CALLS + """
+    for call in (linear, glu):
+        fake.fake_reset()
+        fake.fake_fail_malloc(1)
+        f = lib.eif_hip_qlinear_prep_glu if call is glu else lib.eif_hip_qlinear_prep
+        a = (w.h, C.byref(spec(K))) + (() if call is glu else (None,))
+        assert f(*a, X, N, 4, None) == 0 and fake.fake_launches() == 1
+    """)
