@@ -724,3 +724,56 @@ def test_gemm_tile(gpu, oracle, N, K, g, M):
         assert np.array_equal(y[:, :N].view(np.uint32), oy.view(np.uint32)), bias is None
         assert np.all(y[:, N:] == 7.0)
     qw.close()
+
+
+# Splits along K inside the register-tiled form: N, K, group, M, tokens and rows of its tile, splits.
+TILE_SPLIT = [
+    (130, 1600, 32, 1070, 32, 128, 4),     # 25 steps in 6, 6, 6 and 7; ragged rows
+    (640, 3300, 64, 420, 32, 128, 4),      # 26 steps, a ragged last one
+    (2560, 6912, 96, 230, 32, 128, 3),     # 12 steps a split
+    (2560, 6912, 96, 450, 64, 256, 3),
+    (700, 1700, 32, 1520, 64, 256, 3),     # 9 steps a split
+    (300, 6400, 128, 1520, 64, 256, 4),    # rows past 256, tokens past whole blocks
+    (520, 12700, 256, 419, 32, 128, 4),
+    (1300, 6500, 0, 264, 32, 128, 2),      # one scale per row: 13 steps a split
+    (129, 6400, 0, 1370, 32, 128, 2),
+    (1300, 6500, 0, 970, 64, 256, 2),
+    (520, 6400, 0, 2020, 64, 256, 2),
+]
+
+
+@pytest.mark.parametrize("N,K,g,M", [t[:4] for t in TILE_SPLIT])
+def test_gemm_tile_split(gpu, oracle, N, K, g, M):
+    """The register-tiled GEMM split along K: the bits of the other form with the same split (partial sums added in
+    split order), and with row scales those of the oracle; again on a second call (the tiles' counters are zero), and
+    from the fixed scratch."""
+    import torch
+    lib = gpu.load()
+    w, s = synth.ternary_weight((83, N, K, g), N, K, g)
+    x = synth.activations((84, M, K), M, K, outliers=False)
+    qw = gpu.QWeight(gpu.W_TERNARY, N, K, g, w, s)
+    xq, xs, xq_d, xs_d = dev_inputs(gpu, oracle, x, qw.kpad)
+    bias = torch.from_numpy(synth.rng(85, N).standard_normal(N).astype(np.float32)).to("cuda:0")
+
+    def call(panel, fn="eif_hip_qlinear_ex"):
+        y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda:0")
+        old = lib.eif_hip_set_gemm_panel(panel)
+        try:
+            rc = getattr(lib, fn)(qw.h, gpu.ptr(xq_d), xq_d.stride(0), gpu.ptr(xs_d), gpu.ptr(bias), gpu.ptr(y), N, M, GEMM,
+                                  gpu.stream_ptr())
+        finally:
+            lib.eif_hip_set_gemm_panel(old)
+        assert rc == 0, (fn, rc)
+        torch.cuda.synchronize()
+        return y.cpu().numpy().view(np.uint32)
+
+    want = call(-1)
+    for i in range(2):
+        assert np.array_equal(call(0), want), i
+    assert np.array_equal(call(0, "eif_hip_qlinear_ex_noalloc"), want)
+    if not g:
+        oy = np.zeros((M, N), np.float32)
+        hb = bias.cpu().numpy()
+        oracle.orc_ternary_gemv_rowscale(P(w), P(s), P(xq), qw.kpad, P(xs), P(hb), P(oy), N, M, N, K)
+        assert np.array_equal(want, oy.view(np.uint32))
+    qw.close()
