@@ -535,6 +535,36 @@ def test_prefill_infinite_key(gpu, oracle):
     assert checked >= 3, checked
 
 
+@pytest.mark.parametrize("n,row_scales", [(430, False), (511, False), (300, True)])
+def test_prefill_residual_in_the_gemm(gpu, n, row_scales):
+    """Prompts long enough for the residual add in the GEMM's epilogue (O and down projections, the latter also split along
+    K): keys, values and logits have the bits of the linear followed by the add, which another GEMM form's knob selects."""
+    c = dict(synth.BITNET_2B_DECODE, n_layers=2, vocab=600, seq_len=512)
+    if row_scales:
+        c.update(group_in=0, group_down=0)
+    cfg = synth.bitnet_config(**c)
+    w = synth.bitnet_model((35,), cfg)
+    prompt = [int(t) for t in np.random.default_rng(36).integers(0, cfg["vocab"], n)]
+    lib = gpu.load()
+    m = gpu.BitnetModel(cfg, w)
+
+    def prefilled(panel):
+        old = lib.eif_hip_set_gemm_panel(panel)
+        try:
+            m.reset(prompt)
+            m.prefill(n)
+        finally:
+            lib.eif_hip_set_gemm_panel(old)
+        kv = [a.astype(np.float32).view(np.uint32) for layer in range(2) for a in m.kv_cache(layer, 0, n)]
+        return [m.logits().view(np.uint32)] + kv
+
+    try:
+        want, got = prefilled(-1), prefilled(0)
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    finally:
+        m.close()
+
+
 def test_prefill_then_greedy(gpu, oracle):
     cfg, w = tiny()
     prompt = list(np.random.default_rng(7).integers(0, cfg["vocab"], 12))
