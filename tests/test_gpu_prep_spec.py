@@ -156,9 +156,12 @@ def test_vocab_head_two_step(gpu, oracle, fmt, N, K):
     qw.close()
 
 
-@pytest.mark.parametrize("N,K,M", [(13824, 2560, 1), (512, 640, 3)])
+@pytest.mark.parametrize("N,K,M", [
+    (13824, 2560, 1), (512, 640, 3),
+    (13824, 2560, 3), (13824, 2560, 8), (512, 640, 5),   # the rows prepped in a launch of their own
+])
 def test_glu_form(gpu, oracle, N, K, M):
-    """eif_hip_qlinear_prep_glu: SiLU(gate) * up of the stacked gate|up matrix in one launch. Fed to the next linear
+    """eif_hip_qlinear_prep_glu: SiLU(gate) * up of the stacked gate|up matrix. Fed to the next linear
     with the RMSNorm pre-op, its rows give the bits of the two halves with the SwiGLU pre-op; against the two halves
     it is the SwiGLU of src/eif_tinyllm.c:774-780 to float32 rounding."""
     import torch
@@ -185,6 +188,13 @@ def test_glu_form(gpu, oracle, N, K, M):
     g, u = y2[:, :h].cpu().numpy(), y2[:, h:].cpu().numpy()
     want = (g * (np.float32(1.0) / (np.float32(1.0) + np.exp(-g)))) * u
     got = yg.cpu().numpy()
+    # each row on its own (the prep fused): the same bits
+    y1 = torch.empty((1, h), dtype=torch.float32, device=dev)
+    for m in range(M):
+        sp1 = gpu.prep_spec(x[m:m + 1], pre=1, norm_w=nw, eps=1e-5, block=128, norm=gpu.wht_norm(128))
+        gpu.check(lib.eif_hip_qlinear_prep_glu(qw.h, C.byref(sp1), gpu.ptr(y1), h, 1, gpu.stream_ptr()), "one row")
+        torch.cuda.synchronize()
+        assert np.array_equal(y1.cpu().numpy()[0].view(np.uint32), got[m].view(np.uint32)), m
     assert np.max(np.abs(got - want) / (np.abs(want) + 1e-30 + 1e-6 * np.abs(want).max())) <= 1e-5
     # the down projection: RMSNorm pre-op on the GLU rows == SwiGLU pre-op on the two halves, bit for bit
     blk = 128 if h % 128 == 0 else 64
