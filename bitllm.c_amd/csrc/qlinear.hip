@@ -2488,21 +2488,42 @@ int qlinear_scaled(const eif_hip_qweight *w, const float *scales, const int8_t *
 
 }  // namespace eif
 
-// From kPrepOnceRows token rows on, a linear of FP32 rows preps them in a launch of their own, into the stream's rows
-// buffer, and the GEMV stages the int8 rows: fused, every workgroup preps the rows one after the other (the linears of a
-// BitNet-2B layer, us, fused / prepped: 2 rows 32.3 / 33, 3 rows 41.8 / 33.7, 4 rows 50.9 / 34.0, 8 rows 86.9 / 35.6; the
-// INT4 feed-forward and 151936x1024 head at 3 rows 41.2 / 28.4, at 8 rows 82.1 / 31.8). A short row's prep is a shorter
-// chain, so matrices of up to 1024 columns below the vocabulary sizes go over from kPrepOnceShort rows on (the linears of
-// an INT8 Qwen2.5-0.5B-shaped layer at 3 rows 24.4 / 32.7, at 6 rows 37.5 / 32.5). Codes, scales and sums are the
-// same. gemv(a) launches the GEMV of the prepped rows, or returns 1 where it does not stage the shape; 1 (and the caller
-// takes the fused form) for that, for fewer rows, and where rows_ws() has no buffer.
-constexpr int kPrepOnceRows = 3, kPrepOnceShort = 5;
+// Token rows from which a linear of FP32 rows preps them in a launch of their own, into the stream's rows buffer, and the GEMV
+// stages the int8 rows. Fused, every workgroup preps the rows one after the other: its time grows with the rows, with the
+// length of a row's prep chain (columns, rotation, norm) and, past one workgroup a CU, with the matrix. The two launches take
+// about 8.5 us whatever the shape, most of it the launches. The line lies where the fused form passes that (fused, us a linear,
+// at the rows in front; the two launches take 8.2 to 8.7, from 6912 columns on 9.9):
+//   RMSNorm    2560x512  INT8 7: 8.1, 8: 8.9; rotated 5: 8.0, 6: 9.1     2560x1024 ternary 6: 7.8, 7: 8.7; rotated 5: 8.4, 6: 9.6
+//              2560x1152 INT8 5: 8.3, 6: 9.5; rotated 4: 8.1, 5: 9.4     2560x2048 ternary 5: 8.4, 6: 9.5; rotated 4: 8.4, 5: 10.0
+//              2560x2560 INT8 3: 7.3, 4: 8.7; ternary 4: 8.2, 5: 9.6; rotated 3: 8.4, 4: 10.3
+//              2560x4096 INT8 3: 9.3; ternary 3: 8.3, 4: 10.3; rotated 3: 10.3     2560x6912 ternary 3: 10.0
+//              6912x1024 ternary 5: 7.7, 6: 8.7; rotated 5: 9.3     6912x1536 INT8 3: 8.2, 4: 9.8; ternary 3: 7.6, 4: 9.2;
+//              rotated 3: 9.4     6144x2176 ternary 3: 9.0     6912x2560 INT8 3: 10.7; ternary 3: 9.4; rotated 3: 11.8
+//   no norm    2560x1024 INT8 8: 8.3; ternary 8: 7.6; rotated 8: 8.4     2560x2048 INT8 7: 8.9; ternary 8: 8.2; rotated 7: 8.9
+//              2560x2560 INT8 5: 7.8, 6: 8.8; ternary 6: 8.3, 7: 9.1     2560x4864 INT8 4: 8.8; ternary 4: 8.1, 5: 9.5;
+//              rotated 4: 10.6     6912x1536 INT8 5: 8.0, 6: 8.8; ternary 6: 8.5, 7: 9.3; rotated 5: 9.5
+// INT4 is as fast as ternary. Vocabulary heads are far above the line at 3 rows (the INT4 feed-forward and 151936x1024 head 41.2
+// against 28.4); at 2 rows no shape is (the linears of a BitNet-2B layer 32.3 fused, 33 prepped).
+static int prep_once_rows(const eif_hip_qweight *w, const PrepArgs &p)
+{
+    const int k = w->cols;
+    const bool rot = p.block > 0, i8 = w->fmt == kI8;
+    if (w->rows_pad / 16 >= kBigTiles) return 3;
+    int m;
+    if (rot) m = k <= 1024 ? 6 : k <= 2048 ? 5 : k <= 3072 ? 4 : 3;
+    else m = (k <= 640 ? 8 : k <= 1024 ? 7 : k <= 2048 ? 6 : k <= 3072 ? 5 : k <= 5632 ? 4 : 3) - (i8 && k > 2304 && k <= 5632);
+    if (w->rows >= 6144) m -= k <= 1280 ? 1 : 2;
+    if (p.pre == EIF_HIP_PRE_NONE) m += k > 4096 ? 1 : !i8 && k <= (rot ? 1024 : 2048) ? 3 : 2;
+    return std::max(m, 3);
+}
 
+// The prep of `a`'s rows in a launch of its own, then gemv(a), which launches the GEMV of the prepped rows or returns 1 where it
+// does not stage the shape. Codes, scales and sums are those of the fused form. 1 (and the caller takes the fused form) for
+// that, for fewer rows than prep_once_rows(), and where rows_ws() has no buffer.
 template <class F>
 static int prep_once(const eif_hip_qweight *w, const PrepArgs &p, QArgs a, hipStream_t st, F gemv)
 {
-    const bool brief = w->kpad <= 1024 && w->rows_pad / 16 < kBigTiles;
-    if (a.M < (brief ? kPrepOnceShort : kPrepOnceRows) || !gemv_fits_tile(w)) return 1;
+    if (a.M < prep_once_rows(w, p) || !gemv_fits_tile(w)) return 1;
     const size_t qb = (size_t)a.M * w->kpad;   // a multiple of 16
     if (qb + 4 * (size_t)a.M > kRowsWsBytes) return 1;
     RowsWs *ws = rows_ws(st);
@@ -2608,7 +2629,7 @@ extern "C" int eif_hip_qlinear_prep_glu(const eif_hip_qweight *w, const eif_hip_
     const int kpad = a.nsteps * Geo<kTern, 4>::SC, maxks = 16 / kGluRT;
     int ks = std::min(g_gemv_ksplit > 0 ? g_gemv_ksplit : eif_ceil_div(a.nsteps, 4), maxks);   // as launch_gemv_tiles
     const hipStream_t st = (hipStream_t)stream;
-    if (M >= kPrepOnceRows && kpad <= 8192) {   // what the fused form takes: up to 8 columns on 1024 threads
+    if (kpad <= 8192) {   // what the fused form takes: up to 8 columns on 1024 threads
         int k = ks;
         while (k < maxks && (M * (kpad / 16) > kMaxPieces * 64 * kGluRT * k || a.G > gemv_scl<kTern, 4, true>() * 4 * k)) ++k;
         if (M * (kpad / 16) <= kMaxPieces * 64 * kGluRT * k && a.G <= gemv_scl<kTern, 4, true>() * 4 * k &&

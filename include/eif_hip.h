@@ -106,7 +106,7 @@ int eif_hip_qlinear_acc(const eif_hip_qweight *w, const int8_t *xq, int ldq, int
 
 /* Prep fused into the GEMV: y = linear(prep(x)) for M <= 8 FP32 rows x [M, ldx] of K = cols (K % 32 == 0,
  * rows and signs 16-byte aligned, ldx % 4 == 0, K <= 16384), with the prep contract above (signs, wht_block <= 1024,
- * norm). One launch; from 3 or 5 rows on, by shape, a prep launch into a buffer of the library's and the GEMV, which is
+ * norm). One launch; from 3 to 8 rows on, by shape, a prep launch into a buffer of the library's and the GEMV, which is
  * faster, except inside a graph capture, on hipStreamPerThread and beyond 64 streams: a captured call is one launch that
  * uses no memory but the caller's, so that replays may overlap other work. The result equals eif_hip_prep_rows
  * followed by eif_hip_qlinear bit for bit. M > 8 returns EIF_HIP_E_LIMIT (use the two calls).          */
@@ -138,7 +138,7 @@ typedef struct eif_hip_prep_spec {
 } eif_hip_prep_spec;
 
 /* eif_hip_qlinear_f32 with a pre-op: y = linear(prep(pre(x))) (+ bias). M <= 8 rows: one launch (a row-scaled
- * matrix of 65536 rows or more at M = 1, e.g. a vocabulary head, and from 3 or 5 rows on as eif_hip_qlinear_f32: a
+ * matrix of 65536 rows or more at M = 1, e.g. a vocabulary head, and from 3 to 8 rows on as eif_hip_qlinear_f32: a
  * prep launch, then the GEMV of the prepped rows, with the same output bits); the bias may then be the residual stream
  * itself (y == bias: each output reads its own bias element first). More rows (a prompt batch): the prep of eif_hip_prep_spec_rows into a per-stream
  * workspace, then eif_hip_qlinear on the auto path (the GEMV or the int8-MFMA GEMM by token count and shape),
@@ -147,7 +147,7 @@ typedef struct eif_hip_prep_spec {
 int eif_hip_qlinear_prep(const eif_hip_qweight *w, const eif_hip_prep_spec *spec, const float *bias, float *y,
                          int ldy, int M, void *stream);
 
-/* The gated FFN input of one layer in one GEMV (and a prep launch before it from 3 or 5 rows on, where
+/* The gated FFN input of one layer in one GEMV (and a prep launch before it from 3 rows on, where
  * eif_hip_qlinear_f32 has one): w stacks the gate projection (rows 0 .. rows/2 - 1) over the up projection (rows
  * rows/2 .. rows - 1); y[m, r] = SiLU(g) * u = (g * (1 / (1 + expf(-g)))) * u for r < rows / 2,
  * g and u the outputs eif_hip_qlinear_prep gives for rows r and rows/2 + r (src/eif_tinyllm.c:776-780). Fed to a

@@ -50,14 +50,14 @@ ROWS = [
     # fmt, N, K, group, M, WHT block: calls of 3 to 8 rows, two launches eagerly and one in a capture
     ("tern", 3840, 2560, 128, 4, 128),
     ("tern", 2560, 6912, 96, 8, 128),
-    ("tern", 100, 640, 64, 5, 64),
-    ("tern", 512, 2560, 0, 3, 0),
+    ("tern", 100, 640, 64, 6, 64),
+    ("tern", 512, 2560, 0, 5, 0),
     ("int8", 896, 4864, 0, 3, 0),
     ("int8", 1000, 896, 0, 7, 0),
-    ("int4", 3584, 1024, 0, 6, 0),
+    ("int4", 3584, 1024, 0, 8, 0),
     ("glu", 13824, 2560, 128, 3, 128),
     ("glu", 13824, 2560, 128, 8, 128),
-    ("glu", 512, 640, 128, 5, 0),
+    ("glu", 512, 640, 128, 8, 0),
 ]
 
 

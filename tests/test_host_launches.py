@@ -75,7 +75,7 @@ def test_gated_call_reports_a_failed_prep_launch(fake):
 
 
 ROWS_CALLS = """
-    N, K = 512, 2560
+    N, K = 512, 4096
     w = weight(N, K)
 
     def rows(call, M, st=None):
@@ -103,11 +103,11 @@ def test_rows_buffers(fake):
     """One rows buffer a device and stream, which stays where it is; none for the handle that means a stream per thread;
     64 at most; all given back with the last resident weight."""
     run(fake, ROWS_CALLS + """
-    w2 = weight(256, 4096)
+    w2 = weight(256, 6144)
     live = fake.fake_live()
     _, p = rows(linear, 3)
     assert fake.fake_live() == live + 1
-    assert linear(w2, 256, 4096, 8) == 0 and fake.fake_launches() == 2 and fake.fake_launch_arg1(0) == p
+    assert linear(w2, 256, 6144, 8) == 0 and fake.fake_launches() == 2 and fake.fake_launch_arg1(0) == p
     assert rows(glu, 5)[1] == p and rows(linear, 8, 0x100)[1] != p and fake.fake_live() == live + 2
     fake.fake_device(1)
     assert rows(linear, 4)[1] not in (p, None) and fake.fake_live() == live + 3
@@ -135,4 +135,33 @@ def test_rows_call_without_memory(fake):
         f = lib.eif_hip_qlinear_prep_glu if call is glu else lib.eif_hip_qlinear_prep
         a = (w.h, C.byref(spec(K))) + (() if call is glu else (None,))
         assert f(*a, X, N, 4, None) == 0 and fake.fake_launches() == 1
+    """)
+
+
+@pytest.mark.parametrize("fmt,N,K,block,pre,first", [
+    # the first row count of two launches; 9: none
+    (1, 2560, 512, 0, 1, 8), (1, 2560, 512, 128, 1, 6), (2, 640, 640, 0, 1, 8),
+    (2, 2560, 1024, 0, 1, 7), (1, 6912, 1024, 0, 1, 6), (1, 6912, 1024, 128, 1, 5), (3, 7168, 1024, 0, 1, 6),
+    (2, 2560, 1536, 0, 1, 6), (1, 6912, 1536, 0, 1, 4), (1, 2560, 1536, 128, 1, 5), (1, 4096, 1152, 128, 1, 5),
+    (2, 2560, 2560, 0, 1, 4), (1, 2560, 2560, 0, 1, 5), (1, 2560, 2560, 128, 1, 4), (1, 13824, 2560, 128, 1, 3),
+    (1, 2560, 4096, 0, 1, 4), (2, 2560, 4096, 0, 1, 3), (1, 2560, 6912, 128, 1, 3), (3, 65536, 1024, 0, 1, 3),
+    (1, 2560, 1024, 0, 0, 9), (2, 6912, 1024, 0, 0, 8), (1, 2560, 2048, 128, 0, 7), (2, 2560, 2560, 0, 0, 6),
+    (1, 6912, 2560, 128, 0, 4), (1, 2560, 4864, 0, 0, 5), (3, 65536, 1024, 0, 0, 3),
+])
+def test_rows_where_two_launches_pay(fake, fmt, N, K, block, pre, first):
+    """Rows are prepped in a launch of their own only where that is faster than the fused form, which is a matter of the
+    row's columns, norm and rotation and of the matrix's rows."""
+    run(fake, f"""
+    fmt, N, K, block, first = {fmt}, {N}, {K}, {block}, {first}
+    g = 128 if block else 0
+    if fmt == 1:
+        w = weight(N, K, g)
+    else:
+        w = bh.QWeight(fmt, N, K, 0, np.zeros((N, K if fmt == 2 else K // 2), np.int8), np.ones(N, np.float32))
+    sp = spec(K, block)
+    sp.pre = {pre}
+    for M in range(2, 9):
+        fake.fake_reset()
+        assert lib.eif_hip_qlinear_prep(w.h, C.byref(sp), None, X, N, M, None) == 0
+        assert fake.fake_launches() == (2 if M >= first else 1), M
     """)
