@@ -1,4 +1,4 @@
-// prep_batch.hip -- pre-op, sign flip, blockwise WHT and absmax INT8 of many token rows, one wave a row.
+// prep_batch.hip -- RMSNorm, sign flip, blockwise WHT and absmax INT8 of many token rows, one wave a row.
 //
 // prep_spec_kernel (qlinear.hip) spreads a row over 10 to 16 waves, which suits one row: the chain a wave runs is short.
 // A batch of rows is bound by memory instead, and there most of a workgroup's time was its launch, two barriers and
@@ -27,7 +27,6 @@ __global__ __launch_bounds__(64 * kRowsWg) void prep_batch_kernel(eif::PrepBatch
     if (m >= p.M) return;   // uniform over the wave; no barrier in this kernel
     const int block = LB >= 0 ? (LB > 0 ? 1 << LB : 0) : p.block;
     const float *xr = p.x + (size_t)m * p.ldx;
-    const bool rms = p.pre != EIF_HIP_PRE_NONE;
     float v[NCH][8];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
@@ -40,35 +39,32 @@ __global__ __launch_bounds__(64 * kRowsWg) void prep_batch_kernel(eif::PrepBatch
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[c][e] = 0.0f;
         }
-    float r = 1.0f;
-    if (rms) {
-        // W[w]: the sum of wave w of prep_spec_kernel (256 columns), then the butterfly over its waves
-        static_assert(2 * NCH <= 16, "the waves of its workgroup");
-        float W[16];
+    // W[w]: the sum of wave w of prep_spec_kernel (256 columns), then the butterfly over its waves
+    static_assert(2 * NCH <= 16, "the waves of its workgroup");
+    float W[16];
 #pragma unroll
-        for (int w = 0; w < 16; ++w) W[w] = 0.0f;
+    for (int w = 0; w < 16; ++w) W[w] = 0.0f;
 #pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            float a = 0.0f, b = 0.0f;
+    for (int c = 0; c < NCH; ++c) {
+        float a = 0.0f, b = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) a = fmaf(v[c][e], v[c][e], a), b = fmaf(v[c][4 + e], v[c][4 + e], b);
-            float s = a + b;   // its lanes 2l, 2l + 1
-            s = s + xlane<1>(s);
-            s = s + xlane<2>(s);
-            s = s + xlane<4>(s);   // 8 lanes here, 16 there
-            float q[8];
+        for (int e = 0; e < 4; ++e) a = fmaf(v[c][e], v[c][e], a), b = fmaf(v[c][4 + e], v[c][4 + e], b);
+        float s = a + b;   // its lanes 2l, 2l + 1
+        s = s + xlane<1>(s);
+        s = s + xlane<2>(s);
+        s = s + xlane<4>(s);   // 8 lanes here, 16 there
+        float q[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) q[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), 8 * i));
-            W[2 * c] = ((q[0] + q[1]) + q[2]) + q[3];
-            W[2 * c + 1] = ((q[4] + q[5]) + q[6]) + q[7];
-        }
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1)
-#pragma unroll
-            for (int w = 0; w < 16; w += 2 * o) W[w] = W[w] + W[w + o];
-        const float ss = ((W[0] + 0.0f) + 0.0f) + 0.0f;
-        r = 1.0f / sqrtf(ss / (float)p.K + p.eps);
+        for (int i = 0; i < 8; ++i) q[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), 8 * i));
+        W[2 * c] = ((q[0] + q[1]) + q[2]) + q[3];
+        W[2 * c + 1] = ((q[4] + q[5]) + q[6]) + q[7];
     }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1)
+#pragma unroll
+        for (int w = 0; w < 16; w += 2 * o) W[w] = W[w] + W[w + o];
+    const float ss = ((W[0] + 0.0f) + 0.0f) + 0.0f;
+    const float r = 1.0f / sqrtf(ss / (float)p.K + p.eps);
     auto mul = [&](const float *f) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
@@ -79,7 +75,7 @@ __global__ __launch_bounds__(64 * kRowsWg) void prep_batch_kernel(eif::PrepBatch
             for (int e = 0; e < 8; ++e) v[c][e] = v[c][e] * u[e];
         }
     };
-    if (rms && p.nw) mul(p.nw);
+    if (p.nw) mul(p.nw);
     if (block > 0 && p.signs) mul(p.signs);
     float amax = 0.0f;
 #pragma unroll
@@ -130,13 +126,10 @@ __global__ __launch_bounds__(64 * kRowsWg) void prep_batch_kernel(eif::PrepBatch
     }
 }
 
-template <int NCH>
+template <int NCH, int LB>
 int go(const eif::PrepBatch &p, hipStream_t st)
 {
-    const int grid = eif_ceil_div(p.M, kRowsWg);
-    if (p.block == 128) prep_batch_kernel<NCH, 7><<<grid, 64 * kRowsWg, 0, st>>>(p);
-    else if (p.block == 0) prep_batch_kernel<NCH, 0><<<grid, 64 * kRowsWg, 0, st>>>(p);
-    else prep_batch_kernel<NCH, -1><<<grid, 64 * kRowsWg, 0, st>>>(p);
+    prep_batch_kernel<NCH, LB><<<eif_ceil_div(p.M, kRowsWg), 64 * kRowsWg, 0, st>>>(p);
     EIF_HIP_LAUNCHED();
     return EIF_HIP_OK;
 }
@@ -145,22 +138,33 @@ int go(const eif::PrepBatch &p, hipStream_t st)
 
 namespace eif {
 
-// From kPrepBatchRows rows on: below, the waves of one a row do not fill the chip and a row's chain is what counts. Rows of
-// up to 4096 columns with blocks of up to 256, where prep_spec_kernel holds 4 columns a thread. Longer rows and the
-// SwiGLU pre-op (K = 6912 with it, us, one workgroup a row / one wave a row: 512 rows 9.9 / 21.0, 3001 rows 47.4 / 46.9)
-// stay there: 108 exponentials a lane make the chain too long. K = 2560, RMSNorm, signs, WHT-128: 1024 rows 8.3 / 6.9, 2048
-// 13.7 / 8.1, 3001 18.9 / 10.8 (30 MB read, 8 MB written); without signs and WHT 3001 rows 14.2 / 6.9.
-constexpr int kPrepBatchRows = 768;
-
+// RMSNorm rows where this form is ahead of prep_spec_kernel with 4 columns a thread, which it replaces (kernel times, us,
+// one workgroup a row / one wave a row, inputs rotated past the Infinity Cache):
+// - without rotation from 1024 rows on up to five chunks of columns, from 2048 on up to eight, where a wave's registers
+//   leave fewer of them on a SIMD (K = 896 at 1024 / 3001 rows 4.6 / 4.2, 8.1 / 7.1; 1280 5.4 / 5.3, 9.4 / 8.2; 2048 6.8 /
+//   6.3, 11.2 / 9.8; 2560 8.6 / 7.3, 16.3 / 11.4, at 512 5.3 / 5.6; 3584 at 1500 rows 12.0 / 12.5, at 2048 13.6 / 11.5; 4096
+//   at 1300 rows 11.9 / 12.3, at 2048 14.0 / 12.7);
+// - with rotation for 2305 to 2560 columns from 1024 rows on, where the other form's ten waves a row no longer fill a CU
+//   evenly (K = 2432 at 1024 / 3001 rows 9.9 / 9.2, 19.5 / 15.4; 2560 9.9 / 9.2, 19.5 / 15.8; WHT-64 10.7 / 9.5, 21.5 / 15.6;
+//   2336 with WHT-32 10.3 / 9.0, 20.9 / 14.1). For fewer columns (K = 2304 at 1024 / 2300 rows 8.4 / 9.1, 13.0 / 13.6; 1536
+//   6.6 / 7.2, 10.7 / 11.5) or more (2688 at 1024 rows 9.4 / 10.2, 3584 11.0 / 12.9) a lane's chain of butterflies is too
+//   long for its few waves.
+// Without a norm the two are level; the SwiGLU pre-op's 108 exponentials a lane are too long a chain (K = 6912, 512 rows 9.9 /
+// 21.0, 3001 rows 47.4 / 46.9).
 int launch_prep_batch(const PrepBatch &p, hipStream_t st)
 {
-    if (p.M < kPrepBatchRows || p.pre == EIF_HIP_PRE_SWIGLU_RMS || p.block > 256 || p.ldq > 4096) return 1;
+    if (p.pre != EIF_HIP_PRE_RMS || p.M < 1024 || p.block > 256) return 1;
+    if (p.block > 0) {
+        if (p.ldq <= 2304 || p.ldq > 2560) return 1;
+        return p.block == 128 ? go<5, 7>(p, st) : go<5, -1>(p, st);
+    }
+    if (p.ldq > 4096 || (p.ldq > 2560 && p.M < 2048)) return 1;
     const int nch = eif_ceil_div(p.ldq, 512);
-    if (nch <= 2) return go<2>(p, st);
-    if (nch <= 4) return go<4>(p, st);
-    if (nch <= 5) return go<5>(p, st);
-    if (nch <= 6) return go<6>(p, st);
-    return go<8>(p, st);
+    if (nch <= 2) return go<2, 0>(p, st);
+    if (nch <= 4) return go<4, 0>(p, st);
+    if (nch <= 5) return go<5, 0>(p, st);
+    if (nch <= 6) return go<6, 0>(p, st);
+    return go<8, 0>(p, st);
 }
 
 }  // namespace eif

@@ -12,10 +12,11 @@ struct Launch {
     const void *fn;
     void *stream;
     const void *arg1;   // the kernel's second argument, read as a pointer
+    dim3 grid, block;
 };
 constexpr int kMax = 64;
 Launch g_launch[kMax];
-int g_launches, g_fail_launch = -1, g_fail_malloc, g_mallocs, g_live, g_device, g_capturing;
+int g_launches, g_fail_launch = -1, g_fail_malloc, g_mallocs, g_live, g_device, g_capturing, g_arg1;
 hipError_t g_last;
 dim3 g_grid, g_block;
 size_t g_shmem;
@@ -35,6 +36,9 @@ void fake_reset() { g_launches = 0, g_fail_launch = -1, g_fail_malloc = 0, g_las
 int fake_launches() { return g_launches; }
 void *fake_launch_arg1(int i) { return const_cast<void *>(g_launch[i].arg1); }
 void *fake_launch_stream(int i) { return g_launch[i].stream; }
+int fake_launch_grid(int i) { return (int)g_launch[i].grid.x; }
+int fake_launch_block(int i) { return (int)g_launch[i].block.x; }
+void fake_read_arg1(int on) { g_arg1 = on; }   // only where every launched kernel has a second argument
 void fake_fail_launch(int i) { g_fail_launch = i; }
 void fake_fail_malloc(int on) { g_fail_malloc = on; }
 int fake_mallocs() { return g_mallocs; }
@@ -103,12 +107,12 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shmem, hip
     *grid = g_grid, *block = g_block, *shmem = g_shmem, *st = g_stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *fn, dim3, dim3, void **args, size_t, hipStream_t st)
+hipError_t hipLaunchKernel(const void *fn, dim3 grid, dim3 block, void **args, size_t, hipStream_t st)
 {
     const int i = g_launches++;
     if (i < kMax) {
-        g_launch[i] = {fn, st, nullptr};
-        memcpy(&g_launch[i].arg1, args[1], sizeof(void *));
+        g_launch[i] = {fn, st, nullptr, grid, block};
+        if (g_arg1) memcpy(&g_launch[i].arg1, args[1], sizeof(void *));
     }
     return set(i == g_fail_launch ? hipErrorLaunchFailure : hipSuccess);
 }

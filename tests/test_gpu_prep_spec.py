@@ -219,17 +219,24 @@ def test_glu_form(gpu, oracle, N, K, M):
     (512, 528, 64, 0, False),     # a whole chunk, padding in the next one
     (544, 768, 0, 1, False),
     (2080, 2304, 32, 1, True),
+    (2336, 2336, 32, 1, True),    # just past the rows that one workgroup a row keeps
+    (2400, 2560, 32, 1, False),
     (2560, 2560, 128, 1, True),   # the BitNet layer inputs
+    (2560, 2560, 256, 1, True),
     (2560, 2560, 128, 0, True),
+    (1600, 1664, 0, 1, False),
+    (2304, 2560, 0, 1, False),
+    (2880, 2880, 0, 1, False),
     (3072, 3072, 256, 1, False),
-    (4096, 4096, 128, 1, True),   # the longest row it takes
+    (4064, 4096, 0, 1, False),    # the longest rows it takes
+    (4096, 4096, 128, 1, True),
 ])
 def test_prep_batch_rows(gpu, K, ldq, block, pre, signs):
-    """Batches of 768 rows and more (one wave a row): codes and scales bit for bit those of smaller batches (one
-    workgroup a row), zeros past K, a row of zeros among them."""
+    """Batches of rows on both sides of the rules that give a row one wave: codes and scales bit for bit those of
+    smaller batches (one workgroup a row), zeros past K, a row of zeros among them."""
     import torch
     dev = torch.device("cuda:0")
-    M = 771
+    M = 2051
     x = torch.from_numpy(synth.activations((90, K), M, K)).to(dev)
     x[5] = 0.0
     nw = torch.from_numpy((1.0 + 0.1 * synth.rng(91, K).standard_normal(K)).astype(np.float32)).to(dev)
@@ -244,7 +251,7 @@ def test_prep_batch_rows(gpu, K, ldq, block, pre, signs):
         return xq.cpu().numpy(), xs.cpu().numpy()
 
     q, s = prep(0, M)
-    parts = [prep(0, 400), prep(400, M)]
+    parts = [prep(0, 1000), prep(1000, 1900), prep(1900, M)]
     assert np.array_equal(q, np.concatenate([p[0] for p in parts]))
     assert np.array_equal(s.view(np.uint32), np.concatenate([p[1] for p in parts]).view(np.uint32))
     assert not q[:, K:].any() and not q[5].any() and s[5] == 1.0

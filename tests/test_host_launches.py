@@ -75,6 +75,7 @@ def test_gated_call_reports_a_failed_prep_launch(fake):
 
 
 ROWS_CALLS = """
+    fake.fake_read_arg1(1)
     N, K = 512, 4096
     w = weight(N, K)
 
@@ -164,4 +165,26 @@ def test_rows_where_two_launches_pay(fake, fmt, N, K, block, pre, first):
         fake.fake_reset()
         assert lib.eif_hip_qlinear_prep(w.h, C.byref(sp), None, X, N, M, None) == 0
         assert fake.fake_launches() == (2 if M >= first else 1), M
+    """)
+
+
+@pytest.mark.parametrize("M,K,ldq,pre,block,wave_a_row", [
+    (1023, 2560, 2560, 1, 128, False), (1024, 2560, 2560, 1, 128, True), (3001, 2304, 2304, 1, 128, False),
+    (1024, 2336, 2336, 1, 32, True), (3001, 2688, 2688, 1, 128, False), (3001, 2560, 2560, 1, 512, False),
+    (3001, 2560, 2560, 0, 128, False), (3001, 2560, 2560, 2, 128, False),
+    (1023, 896, 1024, 1, 0, False), (1024, 896, 1024, 1, 0, True), (2047, 2880, 3072, 1, 0, False),
+    (2048, 2880, 3072, 1, 0, True), (3001, 4096, 4096, 1, 0, True), (3001, 4224, 4352, 1, 0, False),
+    (3001, 896, 1024, 0, 0, False),
+])
+def test_prep_of_a_batch(fake, M, K, ldq, pre, block, wave_a_row):
+    """A batch's prep gives a row a wave (workgroups of four rows) only where that is faster than a workgroup a row."""
+    run(fake, f"""
+    M, K, ldq, pre, block = {M}, {K}, {ldq}, {pre}, {block}
+    sp = spec(K, block)
+    sp.pre, sp.x2 = pre, X
+    fake.fake_reset()
+    assert lib.eif_hip_prep_spec_rows(C.byref(sp), K, X, ldq, X, M, None) == 0
+    assert fake.fake_launches() == 1
+    assert (fake.fake_launch_grid(0), fake.fake_launch_block(0) == 256) == \\
+        ((-(-M // 4), True) if {wave_a_row} else (M, fake.fake_launch_block(0) == 256))
     """)
