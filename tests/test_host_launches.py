@@ -9,6 +9,7 @@ import textwrap
 import pytest
 
 from conftest import ROOT
+from test_gpu_qlinear import TILE_SPLIT
 
 LIB = os.path.join(ROOT, "bitllm.c_amd", "libbitllm_hip.so")
 
@@ -187,4 +188,18 @@ def test_prep_of_a_batch(fake, M, K, ldq, pre, block, wave_a_row):
     assert fake.fake_launches() == 1
     assert (fake.fake_launch_grid(0), fake.fake_launch_block(0) == 256) == \\
         ((-(-M // 4), True) if {wave_a_row} else (M, fake.fake_launch_block(0) == 256))
+    """)
+
+
+@pytest.mark.parametrize("N,K,g,M,tm,tn,ks", TILE_SPLIT)
+def test_split_shapes_take_the_tiled_form(fake, N, K, g, M, tm, tn, ks):
+    """The shapes of test_gemm_tile_split run the register-tiled GEMM, with that tile and that many splits."""
+    run(fake, f"""
+    N, K, g, M, tm, tn, ks = {N}, {K}, {g}, {M}, {tm}, {tn}, {ks}
+    w = weight(N, K, g)
+    fake.fake_reset()
+    assert lib.eif_hip_qlinear_ex(w.h, X, w.kpad, X, None, X, N, M, bh.PATH_GEMM, None) == 0
+    tiles = -(-M // tm) * -(-(-(-N // 64) * 64) // tn)
+    assert fake.fake_launches() == 1
+    assert (fake.fake_launch_grid(0), fake.fake_launch_block(0)) == (tiles * ks, 2 * tn)
     """)
