@@ -28,6 +28,19 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 static inline int eif_ceil_div(int a, int b) { return (a + b - 1) / b; }
 static inline int eif_round_up(int a, int b) { return eif_ceil_div(a, b) * b; }
 
+// Compute units of the device that is current at the first call (256 where it cannot be asked).
+inline int eif_device_cus()
+{
+    static const int n = [] {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
+            return 256;
+        return v;
+    }();
+    return n;
+}
+
 // Device-side wave64 reductions (xor butterflies; exact for max and for integers).
 EIF_DEV float eif_wave_max(float v)
 {

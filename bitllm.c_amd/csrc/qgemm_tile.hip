@@ -250,18 +250,6 @@ int go(const TileGemm &g, hipStream_t st)
     return EIF_HIP_OK;
 }
 
-int tile_cus()
-{
-    static const int n = [] {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-            return 256;
-        return v;
-    }();
-    return n;
-}
-
 // Two shapes: "small", 32 tokens x 128 rows on four waves, and "large", 64 tokens x 256 rows on eight (half the
 // decode a token, half the activation reads a row). Small from one workgroup per CU on (row scales: from five eighths of
 // that); below, the forms of qlinear.hip, which split K and give a lone wave shorter chains (us, them / small: g128
@@ -276,7 +264,7 @@ const Shape *pick(const TileGemm &g)
     if (g.fmt != kTern || g.M < 1) return nullptr;
     // the kernel's 32-bit offsets (the other forms refuse such shapes)
     if ((size_t)g.M * g.ldq >= ((size_t)1 << 32) || (size_t)g.rows_pad * g.wld >= ((size_t)1 << 32)) return nullptr;
-    const int C = tile_cus(), small = kSmall.tiles(g) * g.ks, large = kLarge.tiles(g) * g.ks;
+    const int C = eif_device_cus(), small = kSmall.tiles(g) * g.ks, large = kLarge.tiles(g) * g.ks;
     if (8 * small < (g.grouped ? 8 : 5) * C) return nullptr;
     return 2 * large >= 3 * C || (large <= C && 4 * large >= 3 * C) ? &kLarge : &kSmall;
 }

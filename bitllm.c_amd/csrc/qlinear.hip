@@ -10,7 +10,7 @@
 //
 // GPU weight layouts (written once by the repack kernels; same bytes per weight as the reference formats):
 //   ternary, group g = 32*UD: a row is a sequence of steps of 2g columns; a step is 4 slots x UD dwords. Rows lie in
-//     tiles of 16, tile-major (tern_base, Geo::WSTEP): [tile][step][slot][row] of 4*UD bytes, so that the 64 lanes
+//     tiles of 16, tile-major (wt_base, wt_step of qdev.h): [tile][step][slot][row] of 4*UD bytes, so that the 64 lanes
 //     of a wave, which read slot l >> 4 of row l & 15, cover one run of whole cache lines; group scales likewise lie
 //     [tile][group][16 rows].
 //     (Row by row, a load covered 16 half lines 640 bytes or more apart. The linears of a BitNet-2B layer: 23.5 -> 22.8
@@ -1488,18 +1488,6 @@ void count_weight(int d)
     g_nrows = 0;
 }
 
-int device_cus()
-{
-    static const int n = [] {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-            return 256;
-        return v;
-    }();
-    return n;
-}
-
 int g_gemm_split = 0;   // splits along K of the GEMM, 0 = chosen from the shape
 
 // Splits along K (at most 16, at least three steps per split). Fewer tiles than CUs: none for a short K loop
@@ -1515,7 +1503,7 @@ int choose_split(int nsteps, int tiles, bool grouped)
 {
     int ks = g_gemm_split;
     if (ks == 0) {
-        const int C = device_cus();
+        const int C = eif_device_cus();
         if (tiles < C)
             ks = nsteps < 24 ? 1 : std::max(1, std::min((grouped ? 2 : 1) * C / std::max(1, tiles), nsteps / 6));
         else
@@ -1551,7 +1539,7 @@ int gemm_tt(int M, int rt64, int nsteps, bool grouped)
 {
     if (g_gemm_tt > 0) return g_gemm_tt;
     int tt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-    const int C = device_cus();
+    const int C = eif_device_cus();
     auto wgs = [&](int t) { return rt64 * eif_ceil_div(M, 16 * t); };
     // a short K loop takes 32-token tiles below 1.5 workgroups per CU at 64 (ternary 2560x2560 at 512 tokens, 320
     // workgroups: 12.1 us with 32-token tiles, 13.9 with 64; 3840x2560, 480: 15.5 against 14.8; 13824x2560 at 128
@@ -1639,7 +1627,7 @@ size_t gemm_max_lds()
 //   4, 12.7 as a panel).
 int gemm_form(bool grouped, int wgs, int ks, int ns, int wpc)
 {
-    const int C = device_cus();
+    const int C = eif_device_cus();
     const bool resident = wgs <= C * wpc;
     if (!grouped && ks == 1 && wgs > C && wgs <= 4 * C && resident && ns < 8) return -8;
     if (wgs > 2 * C) return 2;
@@ -1862,8 +1850,8 @@ int launch_gemv_s(const QArgs &a, const PrepArgs &p, int rows_pad, int ks, hipSt
     return EIF_HIP_OK;
 }
 
-// The gated form (qgemv_kernel's GLU): fused prep, ternary g128 layout, four row tiles per workgroup (two gate,
-// two up), `half` output rows. E and the waves per tile follow launch_gemv_tiles' rules.
+// The gated form (qgemv_kernel's GLU): prep fused or prepped rows (E = 0), ternary g128 layout, four row tiles per
+// workgroup (two gate, two up), `half` output rows. E and the waves per tile follow launch_gemv_tiles' rules.
 constexpr int kGluRT = 4;
 
 template <int E, int SPW, int LB, int OPS>
@@ -2086,7 +2074,7 @@ int launch_stream_t(const QArgs &a, int rows_pad, const uint8_t *wt, hipStream_t
 {
     const int ldl = NS * Geo<FMT, UD>::SC + 16, ntiles = rows_pad / 16;
     const int wpc = g_gemv_stream > 0 ? g_gemv_stream : kStreamWavesPerCU;
-    const int waves = std::min(ntiles, device_cus() * wpc);
+    const int waves = std::min(ntiles, eif_device_cus() * wpc);
     const int grid = eif_ceil_div(waves, kStreamThreads / 64);
     if (wt)   // the tile-major copy
         qstream_kernel<FMT, UD, ACC, NS, TT, true><<<grid, kStreamThreads, (size_t)a.M * ldl, st>>>(
