@@ -1399,7 +1399,8 @@ int ud_supported(int ud) { return ud == 1 || ud == 2 || ud == 3 || ud == 4 || ud
 
 // Workspaces per (stream, issuing thread): launches that one thread issues on one stream run in order, so one
 // buffer per such pair and purpose suffices, and two threads issuing on the same stream (e.g. the null stream)
-// never share one. Slot 0 the GEMM's split along K, slot 1 the int8 rows of a separate prep. Grown outside graph
+// never share one. Slot 0 the GEMM's split along K, slot 1 the int8 rows of a separate prep (more than kFusedMaxM rows, or
+// the one of a vocabulary head; 3 to 8 rows: rows_ws). Grown outside graph
 // capture (inside a capture a missing buffer returns NULL and the caller takes another path). Buffers are never
 // freed before the process ends, also when replaced by larger ones: a graph captured on the stream keeps using
 // the buffers it was captured with.
@@ -1435,8 +1436,9 @@ float *split_ws(hipStream_t st, size_t bytes, int slot = 0, bool *fresh = nullpt
 
 // The int8 rows and scales of a call of up to kFusedMaxM rows that preps them in a launch of its own (prep_once): one
 // buffer per (device, stream), large enough for every such call, so that it never moves. A call holds `mu` while it issues
-// its two launches: calls of several threads on one stream then follow each other in the stream's order. No buffer inside a
-// capture (replays of a graph run beside other work of its stream and would share it), on hipStreamPerThread (one handle, a
+// its two launches: calls of several threads on one stream then follow each other in the stream's order. (Destroying a
+// stream waits for its work, 46 ms with 46 ms of it queued, so a new stream with its handle finds the buffer free.) No buffer
+// inside a capture (replays of a graph run beside other work of its stream and would share it), on hipStreamPerThread (one handle, a
 // stream per thread), once kRowsWsMax streams have one, or where it cannot be allocated: the caller takes its single
 // launch there. The buffers (8.4 MB at most) are freed with the last resident weight.
 constexpr size_t kRowsWsBytes = kFusedMaxM * (16384 + sizeof(float));

@@ -140,3 +140,33 @@ def test_captured_rows(gpu, fmt, N, K, g, M, block):
     torch.cuda.synchronize()
     assert [np.array_equal(call.bits(), w) for call, w in zip((a, b, c), want)] == [True] * 3
     qw.close()
+
+
+def test_rows_buffer_during_a_capture(gpu):
+    """A stream's first eager call of several rows, while another stream is being captured by the same thread, allocates
+    its rows buffer without ending the capture."""
+    import torch
+    qw = rows_weight(gpu, "tern", 512, 4096, 128)
+    a, b = (RowsCall(gpu, qw, "tern", 4, 128, seed) for seed in (3, 4))
+    a()
+    b()
+    torch.cuda.synchronize()
+    want = [a.bits(), b.bits()]
+    a.y.fill_(float("nan"))
+    b.y.fill_(float("nan"))
+    torch.cuda.synchronize()
+    st, fresh = torch.cuda.Stream(), C.c_void_p()
+    hip = C.CDLL(next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln))
+    assert hip.hipStreamCreateWithFlags(C.byref(fresh), 1) == 0   # not one that an earlier test used
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        a()
+        with torch.cuda.stream(torch.cuda.ExternalStream(fresh.value)):
+            b()
+    torch.cuda.synchronize()
+    assert np.array_equal(b.bits(), want[1])
+    graph.replay()
+    torch.cuda.synchronize()
+    assert np.array_equal(a.bits(), want[0])
+    qw.close()
+    assert hip.hipStreamDestroy(fresh) == 0
