@@ -6,8 +6,10 @@
 //
 // What bounds it: a g128 group costs a wave 4 MFMAs of 32 cycles per 32 x 32 outputs, and 16 conversions, 16 FMAs and
 // the decode's share of vector instructions, which the SIMD overlaps with MFMAs only in part (measured: one MFMA and
-// 12 vector instructions take 60 cycles with two waves on the SIMD, 32 and 26 alone). So the vector unit bounds the
-// group-scaled form, not the matrix cores; four waves per SIMD (128 registers) hide the LDS reads and the barrier of
+// 12 vector instructions take 60 cycles with two waves on the SIMD, 32 and 26 alone). So at thousands of tokens the vector
+// unit bounds the group-scaled form, not the matrix cores (gate|up 13824x2560 at 3001 tokens: vector instructions in 66% of the
+// cycles, MFMAs in 35%, half of these beside vector instructions); at 512 tokens (40 and 22%) and with row scales it is the
+// chain of a step and the ends of a launch. Four waves per SIMD (128 registers) hide the LDS reads and the barrier of
 // each step. Measured (us, one launch; the forms of qlinear.hip against this one): g128 13824x2560 at 512 / 3001 tokens
 // 37.8 / 229 against 28.2 / 159, 3840x2560 at 512 / 3001 15.3 / 59 against 12.3 / 44.7; g96 2560x6912 at 3001 tokens 163
 // against 79.6; row scales 13824x2560 at 200 / 3001 tokens 20.7 / 193 against 13.1 / 116.
