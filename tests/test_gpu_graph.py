@@ -170,3 +170,37 @@ def test_rows_buffer_during_a_capture(gpu):
     assert np.array_equal(a.bits(), want[0])
     qw.close()
     assert hip.hipStreamDestroy(fresh) == 0
+
+
+def test_rows_calls_of_two_threads(gpu):
+    """Two threads that issue calls of several rows on one stream share its rows buffer and keep to their own rows."""
+    import threading
+
+    import torch
+    qw = rows_weight(gpu, "tern", 512, 4096, 128)
+    calls = [RowsCall(gpu, qw, "tern", 8, 128, seed) for seed in (5, 6)]
+    for call in calls:
+        call()
+    torch.cuda.synchronize()
+    want = [call.bits() for call in calls]
+    outs = [[torch.full_like(call.y, float("nan")) for _ in range(40)] for call in calls]
+    failed = []
+
+    def issue(call, ys):
+        try:
+            for y in ys:
+                call.y = y
+                call()
+        except BaseException as e:   # an assertion in a thread is not the test's own
+            failed.append(e)
+
+    threads = [threading.Thread(target=issue, args=a) for a in zip(calls, outs)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not failed
+    for ys, w in zip(outs, want):
+        assert all(np.array_equal(y.cpu().numpy().view(np.uint32), w) for y in ys)
+    qw.close()
