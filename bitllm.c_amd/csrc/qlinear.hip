@@ -2494,34 +2494,38 @@ int qlinear_scaled(const eif_hip_qweight *w, const float *scales, const int8_t *
 //              rotated 4: 10.6     6912x1536 INT8 5: 8.0, 6: 8.8; ternary 6: 8.5, 7: 9.3; rotated 5: 9.5
 // INT4 is as fast as ternary. Vocabulary heads are far above the line at 3 rows (the INT4 feed-forward and 151936x1024 head 41.2
 // against 28.4); at 2 rows no shape is (the linears of a BitNet-2B layer 32.3 fused, 33 prepped).
+constexpr int kPrepOnceMin = 3;
+
 static int prep_once_rows(const eif_hip_qweight *w, const PrepArgs &p)
 {
     const int k = w->cols;
     const bool rot = p.block > 0, i8 = w->fmt == kI8;
-    if (w->rows_pad / 16 >= kBigTiles) return 3;
+    if (w->rows_pad / 16 >= kBigTiles) return kPrepOnceMin;
     int m;
     if (rot) m = k <= 1024 ? 6 : k <= 2048 ? 5 : k <= 3072 ? 4 : 3;
     else m = (k <= 640 ? 8 : k <= 1024 ? 7 : k <= 2048 ? 6 : k <= 3072 ? 5 : k <= 5632 ? 4 : 3) - (i8 && k > 2304 && k <= 5632);
     if (w->rows >= 6144) m -= k <= 1280 ? 1 : 2;
     if (p.pre == EIF_HIP_PRE_NONE) m += k > 4096 ? 1 : !i8 && k <= (rot ? 1024 : 2048) ? 3 : 2;
-    return std::max(m, 3);
+    return std::max(m, kPrepOnceMin);
 }
 
-// The prep of `a`'s rows in a launch of its own, then gemv(a), which launches the GEMV of the prepped rows or returns 1 where it
+// The prep of `rows` in a launch of its own, then gemv(a), which launches the GEMV of the prepped rows or returns 1 where it
 // does not stage the shape. Codes, scales and sums are those of the fused form. 1 (and the caller takes the fused form) for
 // that, for fewer rows than prep_once_rows(), and where rows_ws() has no buffer.
 template <class F>
-static int prep_once(const eif_hip_qweight *w, const PrepArgs &p, QArgs a, hipStream_t st, F gemv)
+static int prep_once(const eif_hip_qweight *w, const PrepArgs &p, const QArgs &rows, hipStream_t st, F gemv)
 {
-    if (a.M < prep_once_rows(w, p) || !gemv_fits_tile(w)) return 1;
-    const size_t qb = (size_t)a.M * w->kpad;   // a multiple of 16
-    if (qb + 4 * (size_t)a.M > kRowsWsBytes) return 1;
+    const int M = rows.M;
+    if (M < kPrepOnceMin || M < prep_once_rows(w, p) || !gemv_fits_tile(w)) return 1;
+    const size_t qb = (size_t)M * w->kpad;   // a multiple of 16
+    if (qb + 4 * (size_t)M > kRowsWsBytes) return 1;
     RowsWs *ws = rows_ws(st);
     if (!ws) return 1;
     std::lock_guard<std::mutex> lk(ws->mu);
     float *xs = reinterpret_cast<float *>(ws->p + qb);
-    const int rc = launch_prep_spec(p, ws->p, w->kpad, xs, a.M, st);
+    const int rc = launch_prep_spec(p, ws->p, w->kpad, xs, M, st);
     if (rc) return rc == EIF_HIP_E_LIMIT ? 1 : rc;
+    QArgs a = rows;
     a.xq = ws->p, a.ldq = w->kpad, a.xs = xs;
     return gemv(a);
 }
